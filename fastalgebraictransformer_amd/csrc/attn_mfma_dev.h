@@ -304,7 +304,7 @@ template <int D> __device__ __forceinline__ int eoff(int row, int col) {
 __device__ __forceinline__ void epi_put(short* tile, int off, uint32_t lo, uint32_t hi) {
   *reinterpret_cast<u32x2*>(tile + off) = u32x2{lo, hi};
 }
-// rows 0 .. R - 1 of the tile to base[(row0 + r) * stride], rows with
+// rows r = rbase .. rbase + R - 1 of the tile to base[(row0 + r) * stride], rows with
 // row0 + r >= nrows and columns at or past cols skipped; the tile must be complete (written by this wave,
 // with a barrier or an LDS wait in between). Non-temporal stores: the outputs
 // are not re-read by the kernel that writes them, and write-back stores left
@@ -313,11 +313,12 @@ __device__ __forceinline__ void epi_put(short* tile, int off, uint32_t lo, uint3
 // shape, forward 0.5%).
 template <typename T, int D, int R>
 __device__ __forceinline__ void epi_rows_out(const short* tile, int lane, T* __restrict__ base, int64_t stride,
-                                             int row0, int nrows, int cols = D) {
+                                             int row0, int nrows, int cols = D, int rbase = 0) {
   constexpr int CPR = D / 8, RPI = 64 / CPR;  // chunks per row, rows per instruction
+  static_assert(R % RPI == 0, "whole instructions");
 #pragma unroll
   for (int i = 0; i < R / RPI; ++i) {
-    const int r = i * RPI + lane / CPR, c = lane % CPR;
+    const int r = rbase + i * RPI + lane / CPR, c = lane % CPR;
     const i16x8 v = *reinterpret_cast<const i16x8*>(tile + eoff<D>(r, 8 * c));
     if (row0 + r < nrows && 8 * c < cols)
       __builtin_nontemporal_store(v, reinterpret_cast<i16x8*>(base + (int64_t)(row0 + r) * stride + 8 * c));

@@ -106,22 +106,48 @@ constexpr int kModeKeyMask = 2;
 // D <= 128: 4-wave blocks, two per CU. D = 256: the K and V tiles take 128 KB
 // of LDS, so one block per CU of 8 waves (two per SIMD), 16 queries per wave
 // (the Q fragments and O accumulators of 16 queries take 96 VGPRs).
+//
+// KG = 2 (small grids, fwd_split_keys): the block's waves form two key groups,
+// each taking 32 of a tile's 64 keys for half as many queries (64 per block
+// instead of 128). A lone block on a CU has one wave per SIMD and is bound by
+// that wave's own chain of MFMAs, VALU work and LDS waits (1.33 us per key tile
+// at D = 128); the split halves the chain (0.8 us), doubles the blocks and
+// evens out the causal triangle, at twice the tile loads per query and one
+// exchange of the two groups' sums at the end (plain additions: no running
+// maximum; a fixed order, so deterministic). Measured (bf16, causal, GPU time):
+// B=1, H=16, T=1999, D=128 46 -> 30 us; B=4, H=12, T=777, D=64 17.0 -> 11.3;
+// B=1, H=12, T=2048, D=64 37 -> 22; B=2, H=12, T=512, D=64 12.0 -> 8.0. Also
+// measured: four key groups on 128-key tiles (8 waves, half the CU's blocks)
+// 20-60% slower than two wherever more than one block per CU runs, and 8 waves
+// of 16 queries 3-15% slower at D = 128 (twice the LDS reads per MFMA).
+// Those blocks are mostly all resident at once, so a CU's time is the sum of
+// the blocks it is given: `snake` runs every second round of 256 blocks
+// (32 per XCD) backwards, so that a CU's long causal blocks come with short
+// ones (B=4, H=12, T=777, D=64 12.4 -> 11.3 us, the T=1999 call 31.7 -> 30.3).
 // ============================================================================
-template <typename T, int D, int MODE, int QS, int NW = kNW, int DE = D>
-__global__ __launch_bounds__(64 * NW, NW == 4 && QS == 2 ? 2 : 1) void attn_fwd_k(AttnArgs a) {
+template <typename T, int D, int MODE, int QS, int NW = kNW, int DE = D, int KG = 1>
+__global__ __launch_bounds__(64 * NW, NW == 4 && QS == 2 ? 2 : 1) void attn_fwd_k(AttnArgs a, int snake) {
   typedef Mfma<T> M;
+  static_assert(KG == 1 || KG == 2, "key groups");
   constexpr int KK = DE / 32;  // k-steps of QK^T
   constexpr int DS = DE / 16;  // 16-wide d subtiles of O^T
   constexpr bool kCausal = (MODE & kModeCausal) != 0;
   constexpr bool kKM = (MODE & kModeKeyMask) != 0;
   constexpr int RW = 16 * QS;    // queries per wave
-  constexpr int BMQ = NW * RW;  // queries per block
+  constexpr int QG = NW / KG;   // query groups (waves of one key group)
+  constexpr int BMQ = QG * RW;  // queries per block
   __shared__ short sk[2][kBN * D];
   __shared__ short sv[2][kBN * D];
 
   const int T_ = a.T, H = a.H;
   int bh, rank;
-  block_order((int)blockIdx.x, a.B * H, bh, rank);
+  int id = (int)blockIdx.x;
+  if (KG == 2 && snake) {  // round r of 256 blocks backwards: odd, whole, resident from the start
+    const int sl = id >> 3, r = sl >> 5;
+    if ((r & 1) && r < (int)gridDim.x / 256 && r < (D == 128 ? 2 : 4))
+      id = (id & 7) | ((32 * r + 31 - (sl & 31)) << 3);
+  }
+  block_order(id, a.B * H, bh, rank);
   const int n_qt = (T_ + BMQ - 1) / BMQ;
   const int q0 = (n_qt - 1 - rank) * BMQ;
   const int b = bh / H, h = bh - b * H;
@@ -129,7 +155,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && QS == 2 ? 2 : 1) void attn_fwd_
   // forward measured 3% slower
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 4, li = lane & 15;
-  const int qw = q0 + RW * w;
+  const int qw = q0 + RW * (KG == 1 ? w : w % QG);
+  // the wave's part of every key tile: rows hk .. hk + TK - 1
+  constexpr int TK = kBN / KG;
+  const int hk = KG == 1 ? 0 : TK * (w / QG);
 
   const T* qp = (const T*)a.q + b * a.sq[0] + h * a.sq[1];
   const T* kp = (const T*)a.k + b * a.sk[0] + h * a.sk[1];
@@ -161,7 +190,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && QS == 2 ? 2 : 1) void attn_fwd_
   // place) from the first tile wholly above it on
   f32x4 cbx = cb;
   float sgn = 1.f;
-  // key validity of the current tile (bit r: key k0 + r), and its first key
+  // key validity of the wave's TK keys of the current tile (bit r: key kcur + r)
+  constexpr uint64_t kAll = TK == 64 ? ~0ull : (1ull << (TK & 63)) - 1ull;
   uint64_t vm = ~0ull;
   int kcur = 0;
   const uint8_t* kmb = kKM ? a.km + (int64_t)b * a.skm : nullptr;
@@ -175,7 +205,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && QS == 2 ? 2 : 1) void attn_fwd_
 #pragma unroll
   for (int qs = 0; qs < QS; ++qs) lsum[qs] = 0.f;
 
-  TileDma<D, NW> dk, dv;
+  TileDma<D, NW, kBN> dk, dv;
   dk.init(w, lane, sk2, DR);
   dv.init(w, lane, sv2, DR);
 
@@ -235,19 +265,22 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && QS == 2 ? 2 : 1) void attn_fwd_
       for (int qs = 0; qs < QS; ++qs) oacc[ds][qs] = M::mma(vt, pf[qs], oacc[ds][qs]);
     }
   };
+  // k0, ks_, vs_: the wave's first key of the tile and its rows
   auto tile = [&](auto masked_tag, int k0, const short* ks_, const short* vs_) __attribute__((always_inline)) {
     f32x4 sA[QS], sB[QS];
     uint32_t pa0[QS][2], pb0[QS][2], pa1[QS][2], pb1[QS][2];
     m1(0, sA, ks_);
     m1(16, sB, ks_);
     vh(masked_tag, k0, sA, pa0);
-    m1(32, sA, ks_);
+    if constexpr (KG == 1) m1(32, sA, ks_);
     vh(masked_tag, k0 + 16, sB, pb0);
     m2(0, pa0, pb0, vs_);
-    m1(48, sB, ks_);
-    vh(masked_tag, k0 + 32, sA, pa1);
-    vh(masked_tag, k0 + 48, sB, pb1);
-    m2(32, pa1, pb1, vs_);
+    if constexpr (KG == 1) {
+      m1(48, sB, ks_);
+      vh(masked_tag, k0 + 32, sA, pa1);
+      vh(masked_tag, k0 + 48, sB, pb1);
+      m2(32, pa1, pb1, vs_);
+    }
   };
   // which variant a tile takes. Causal without a padding mask: below the
   // diagonal plain, straddling it masked, above it skipped. Otherwise a tile
@@ -257,23 +290,23 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && QS == 2 ? 2 : 1) void attn_fwd_
   // first tile wholly above the diagonal.
   auto tile_step = [&](int k0, const short* ks_, const short* vs_) __attribute__((always_inline)) {
     if constexpr (kCausal && !kKM) {
-      if (k0 + kBN - 1 <= qw)
+      if (k0 + TK - 1 <= qw)
         tile(std::false_type{}, k0, ks_, vs_);
       else if (k0 <= qw + RW - 1)
         tile(std::true_type{}, k0, ks_, vs_);
     } else {
       bool plain;
       if constexpr (kCausal) {
-        plain = k0 + kBN - 1 <= qw;
+        plain = k0 + TK - 1 <= qw;
       } else {
         const bool above = k0 > qw + RW - 1;
         if (above && sgn > 0.f) {
           cbx = -cbx;
           sgn = -1.f;
         }
-        plain = above || k0 + kBN - 1 <= qw;
+        plain = above || k0 + TK - 1 <= qw;
       }
-      plain = plain && vm == ~0ull;
+      plain = plain && vm == kAll;
       if (vm == 0ull || (kCausal && k0 > qw + RW - 1)) {
       } else if (plain) {
         tile(std::false_type{}, k0, ks_, vs_);
@@ -283,11 +316,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && QS == 2 ? 2 : 1) void attn_fwd_
     }
   };
 
-  const int n_kt = kCausal ? (std::min(q0 + BMQ, T_) + kBN - 1) / kBN : (T_ + kBN - 1) / kBN;
-  // this lane's padding-mask byte of key tile kt (0 past the end)
+  const int n_kt = ((kCausal ? std::min(q0 + BMQ, T_) : T_) + kBN - 1) / kBN;
+  // this lane's padding-mask byte of the wave's keys of tile kt (0 past the end)
   auto kmbyte = [&](int kt) __attribute__((always_inline)) {
-    const int j = kt * kBN + lane;
-    return (kKM && j < T_) ? (uint32_t)kmb[j] : 0u;
+    const int j = kt * kBN + hk + lane;
+    return (kKM && j < T_ && (TK == 64 || lane < TK)) ? (uint32_t)kmb[j] : 0u;
   };
   uint32_t kmn = kmbyte(0);  // loaded one tile ahead of its use
   dk.issue(sk[0], kp, kbytes, 0, sk2, w);
@@ -303,15 +336,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && QS == 2 ? 2 : 1) void attn_fwd_
       dk.issue(sk[buf ^ 1], kp, kbytes, (kt + 1) * kBN, sk2, w);
       dv.issue(sv[buf ^ 1], vp, vbytes, (kt + 1) * kBN, sv2, w);
     }
-    const int k0 = kt * kBN;
+    const int k0 = kt * kBN + hk;
     kcur = k0;
     if constexpr (kKM) {
       vm = __builtin_amdgcn_ballot_w64(kmn != 0u);
       if (kt + 1 < n_kt) kmn = kmbyte(kt + 1);
     } else if constexpr (!kCausal) {
-      vm = T_ - k0 >= kBN ? ~0ull : (1ull << (T_ - k0)) - 1ull;
+      const int left = T_ - k0;
+      vm = left >= TK ? kAll : left <= 0 ? 0ull : (1ull << left) - 1ull;
     }
-    tile_step(k0, sk[buf], sv[buf]);
+    tile_step(k0, sk[buf] + hk * D, sv[buf] + hk * D);
     dma_wait();
     __syncthreads();
   };
@@ -320,29 +354,71 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && QS == 2 ? 2 : 1) void attn_fwd_
     if (kt + 1 < n_kt) step(kt + 1, std::integral_constant<int, 1>{});
   }
 
-  // epilogue: L' across the 4 lane groups, normalise; O through the wave's
-  // own RW x D staging tile in the (now idle) K buffers, stored by rows
+  // epilogue: L' across the 4 lane groups, normalise; O through the query
+  // group's RW x D staging tile in the (now idle) K buffers, stored by rows
   T* __restrict__ op = (T*)a.o + b * a.so[0] + h * a.so[1];
   float* __restrict__ Lp = a.L + b * a.sl[0] + h * a.sl[1];
-  static_assert(sizeof(sk) >= NW * RW * D * 2, "staging tiles fit the K buffers");
-  short* const et = &sk[0][0] + w * RW * D;
+  static_assert(sizeof(sk) >= QG * RW * D * 2, "staging tiles fit the K buffers");
+  short* const et = &sk[0][0] + (KG == 1 ? w : w % QG) * RW * D;
 #pragma unroll
   for (int qs = 0; qs < QS; ++qs) {
-    float l = lsum[qs];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    const int qrow = qw + 16 * qs + li;
-    const float inv = 1.f / (l + 16.f * a.eps);
-    if (qrow < T_ && g == 0) Lp[(int64_t)qrow * a.sl[2]] = l * 0.0625f;
+    lsum[qs] += __shfl_xor(lsum[qs], 16, 64);
+    lsum[qs] += __shfl_xor(lsum[qs], 32, 64);
+  }
+  // one 16 x 16 piece (d subtile ds, query subtile qs) of O^T, normalised
+  auto put = [&](int ds, int qs, const f32x4& o) __attribute__((always_inline)) {
+    const float inv = 1.f / (lsum[qs] + 16.f * a.eps);
+    epi_put(et, eoff<D>(16 * qs + li, 16 * ds + 4 * g), M::pack2(o[0] * inv, o[1] * inv),
+            M::pack2(o[2] * inv, o[3] * inv));
+  };
+  if constexpr (KG == 1) {
 #pragma unroll
-    for (int ds = 0; ds < DS; ++ds) {
-      const f32x4 o = oacc[ds][qs];
-      epi_put(et, eoff<D>(16 * qs + li, 16 * ds + 4 * g), M::pack2(o[0] * inv, o[1] * inv),
-              M::pack2(o[2] * inv, o[3] * inv));
+    for (int ds = 0; ds < DS; ++ds)
+#pragma unroll
+      for (int qs = 0; qs < QS; ++qs) put(ds, qs, oacc[ds][qs]);
+  } else {
+    // the two waves of a query group exchange halves of their sums through the
+    // (idle) tile buffers: wave kg keeps the d subtiles [kg DK, (kg + 1) DK)
+    // and adds the other wave's part of them; both add up L'
+    constexpr int DK = DS / 2;
+    static_assert(DS % 2 == 0 && sizeof(sv) >= (size_t)NW * DK * QS * 1024 && sizeof(sk) >= (size_t)NW * QS * 256,
+                  "the exchange fits the tile buffers");
+    const int kg = w / QG, wo = (w + QG) % NW;  // wo: the other wave
+    f32x4* const xo = reinterpret_cast<f32x4*>(&sv[0][0]);
+    float* const xl = reinterpret_cast<float*>(&sk[0][0]);
+    f32x4 os[DK][QS];
+#pragma unroll
+    for (int d = 0; d < DK; ++d)
+#pragma unroll
+      for (int qs = 0; qs < QS; ++qs) {
+        os[d][qs] = kg ? oacc[DK + d][qs] : oacc[d][qs];
+        xo[((w * DK + d) * QS + qs) * 64 + lane] = kg ? oacc[d][qs] : oacc[DK + d][qs];
+      }
+#pragma unroll
+    for (int qs = 0; qs < QS; ++qs) xl[(w * QS + qs) * 64 + lane] = lsum[qs];
+    __syncthreads();
+#pragma unroll
+    for (int qs = 0; qs < QS; ++qs) {
+      lsum[qs] += xl[(wo * QS + qs) * 64 + lane];
+#pragma unroll
+      for (int d = 0; d < DK; ++d) os[d][qs] += xo[((wo * DK + d) * QS + qs) * 64 + lane];
     }
+    __syncthreads();  // the sums are read: the K buffers become staging tiles
+#pragma unroll
+    for (int d = 0; d < DK; ++d)
+#pragma unroll
+      for (int qs = 0; qs < QS; ++qs) put(kg * DK + d, qs, os[d][qs]);
+  }
+#pragma unroll
+  for (int qs = 0; qs < QS; ++qs) {
+    const int qrow = qw + 16 * qs + li;
+    if (qrow < T_ && g == 0 && (KG == 1 || w < QG)) Lp[(int64_t)qrow * a.sl[2]] = lsum[qs] * 0.0625f;
   }
   __syncthreads();  // orders the tile's writes before its reads
-  epi_rows_out<T, D, RW>(et, lane, op, a.so[2], qw, T_, DR);
+  // whole rows, RO of them per wave (at least one store instruction's)
+  constexpr int RO = std::max(RW / KG, 512 / D);
+  if (KG == 1 || (w / QG) * RO < RW)
+    epi_rows_out<T, D, RO>(et, lane, op, a.so[2], qw, T_, DR, KG == 1 ? 0 : (w / QG) * RO);
 }
 
 // Everything the backward's MFMA kernels take besides the inputs (the
@@ -1411,10 +1487,42 @@ inline BwdWs bwd_ws(void* base, int64_t B, int64_t H, int64_t T, int64_t D, bool
   return w;
 }
 
+// Whether a forward over nb blocks of 128 queries runs the key-split kernel
+// (KG = 2) instead. The one-group kernel holds two blocks per CU at D = 128 and
+// four at D <= 64, and is the faster one once the grid fills them (fewer tile
+// loads per query); the split wins below that, in causal mode the longer T is
+// the nearer to a full grid, since it also evens out the triangle. Measured,
+// one group / split: D = 128, nb = 256: T=256 11.0 / 9.6 us, T=512 16.5 / 12.9,
+// T=1024 25.6 / 18.3; nb = 384: T=512 16.6 / 17.7, T=768 23.0 / 21.0, T=1024
+// 27.8 / 24.8; nb = 512: T=512 17.5 / 20.9, T=1024 29.3 / 29.3, T=2048 53.0 /
+// 48.0, T=4096 98 / 86; nb = 768: T=2048 68.8 / 72.1; nb = 256, T=128 8.1 / 8.5.
+// D = 64: nb = 768: T=512 17.8 / 16.1, T=2048 48.5 / 42.7; nb = 960: T=512
+// 19.6 / 20.6, T=2048 59.3 / 51.0; nb = 1024: T=8192 207 / 185; nb = 3072,
+// T=2048 162 / 185. Non-causal: D = 128, nb = 256 48.5 / 45.5, nb = 320 69.8 /
+// 69.4, nb = 384 39.6 / 40.5; D = 64, nb = 384 31.1 / 26.0, nb = 512 30.6 / 31.7.
+inline bool fwd_split_keys(int D, bool causal, int64_t nb, int64_t T) {
+  const int64_t cus = num_cus();
+  if (D > 128) return false;
+  if (!causal) return 2 * nb <= (D == 128 ? 2 : 3) * cus;
+  if (D == 128) return T > 128 ? nb * 512 <= cus * std::min<int64_t>(std::max<int64_t>(T, 512), 1024) : 2 * nb <= cus;
+  return nb * 256 <= cus * std::min<int64_t>(std::max<int64_t>(T, 768), 1024);
+}
+
 template <typename T, int D, int DE, int MODE> int launch_fwd(const AttnArgs& a, hipStream_t st) {
   constexpr int QS = D == 256 ? 1 : kFwdQS, NW = D == 256 ? 8 : kNW, BMQ = NW * 16 * QS;
   const int64_t nb = (int64_t)((a.T + BMQ - 1) / BMQ) * a.B * a.H;
-  hipLaunchKernelGGL((attn_fwd_k<T, D, MODE, QS, NW, DE>), dim3((unsigned)nb), dim3(64 * NW), 0, st, a);
+  if constexpr (D <= 128) {
+    if (fwd_split_keys(D, (MODE & kModeCausal) != 0, nb, a.T)) {
+      constexpr int BQ2 = BMQ / 2;
+      const int64_t nb2 = (int64_t)((a.T + BQ2 - 1) / BQ2) * a.B * a.H;
+      // past ~5 rounds at D <= 64 (four resident) the later rounds' dynamic
+      // placement does better without (B=5, H=12, T=2048 51.0 against 52.9 us)
+      const int snake = (MODE & kModeCausal) != 0 && (D == 128 || nb2 <= 5 * (int64_t)num_cus());
+      hipLaunchKernelGGL((attn_fwd_k<T, D, MODE, QS, NW, DE, 2>), dim3((unsigned)nb2), dim3(64 * NW), 0, st, a, snake);
+      return check_launch("kat_attn_fwd (mfma, split keys)");
+    }
+  }
+  hipLaunchKernelGGL((attn_fwd_k<T, D, MODE, QS, NW, DE>), dim3((unsigned)nb), dim3(64 * NW), 0, st, a, 0);
   return check_launch("kat_attn_fwd (mfma)");
 }
 
