@@ -4,11 +4,11 @@
 // Design (MI355X): these ops do a handful of flops per byte, so the only
 // roofline that matters is HBM (8 TB/s). Every kernel touches each tensor
 // exactly once:
-//   * row-resident kernels (softmax, norm): a 256-thread block owns a row at a
-//     time, holds it in registers as packed 16-byte vectors, reduces with
-//     wavefront shuffles plus a 4-entry LDS exchange and writes the result --
-//     one HBM pass where the reference makes two (fused_ops.py:74-106,
-//     319-342, 395-423);
+//   * row-resident kernels (softmax, norm): a 256-thread block (or, for narrow
+//     rows, one wave) owns a row at a time, holds it in registers as packed
+//     16-byte vectors, reduces with wavefront shuffles (plus a 4-entry LDS
+//     exchange across a block) and writes the result -- one HBM pass where the
+//     reference makes two (fused_ops.py:74-106, 319-342, 395-423);
 //   * SwiGLU is a flat elementwise stream of 16-byte vectors with row strides,
 //     so gate/value can be the two halves of one packed buffer;
 //   * the norm backward folds the weight gradient (torch ops at
@@ -300,35 +300,43 @@ template <typename A> __device__ __forceinline__ A block_sum_par(A v, A (*red)[k
   return (red[par][0] + red[par][1]) + (red[par][2] + red[par][3]);
 }
 
+// Sum over a row's threads: the block's 256, or one wave's 64 (no barrier)
+template <int TPR, typename A> __device__ __forceinline__ A row_sum(A v, A (*red)[kRowWaves], int par) {
+  if constexpr (TPR == 256) return block_sum_par(v, red, par);
+  else return wave_sum(v);
+}
+
 // Loads this thread's chunks of one row. Chunks past the row end re-read the
 // row's first chunk (always in bounds) and are masked where they are used:
 // a conditional load here would compile to a branch that waits for the data
 // on the spot, serialising the prefetch.
 // FULL: the row is exactly NCH chunk rounds long, so every chunk is in range
 // and the column tests fold away (the norm kernels take this when it holds).
-template <typename T, int NCH, bool FULL = false>
+// TPR: threads per row, 256 (the block's) or 64 (one wave's).
+template <int TPR> __device__ __forceinline__ int row_tid() { return (int)threadIdx.x & (TPR - 1); }
+template <typename T, int NCH, bool FULL = false, int TPR = 256>
 __device__ __forceinline__ void load_row(const T* __restrict__ base, int n_cols, VecT<T, Raw<T>::V> (&r)[NCH]) {
   constexpr int V = Raw<T>::V;
 #pragma unroll
   for (int k = 0; k < NCH; ++k) {
-    const int col = ((int)threadIdx.x + 256 * k) * V;
+    const int col = (row_tid<TPR>() + TPR * k) * V;
     r[k] = ld_vec<T, V>(base + ((FULL || col < n_cols) ? col : 0));
   }
 }
-template <bool FULL = false> __device__ __forceinline__ bool chunk_in(int k, int V, int n_cols) {
-  return FULL || ((int)threadIdx.x + 256 * k) * V < n_cols;
+template <bool FULL = false, int TPR = 256> __device__ __forceinline__ bool chunk_in(int k, int V, int n_cols) {
+  return FULL || (row_tid<TPR>() + TPR * k) * V < n_cols;
 }
 
 // The weight values of this thread's chunks, with 16-byte loads (the caller
 // checks 16-byte alignment of w); out-of-row chunks read chunk 0.
-template <typename T, typename W, int NCH>
+template <typename T, typename W, int NCH, int TPR = 256>
 __device__ __forceinline__ void load_weight(const W* __restrict__ w, int n_cols,
                                             typename AccT<T>::type (&wv)[NCH][Raw<T>::V]) {
   constexpr int V = Raw<T>::V;
   constexpr int PER = 16 / (int)sizeof(W);  // weights per 16-byte load
 #pragma unroll
   for (int k = 0; k < NCH; ++k) {
-    const int col = ((int)threadIdx.x + 256 * k) * V;
+    const int col = (row_tid<TPR>() + TPR * k) * V;
     const W* base = w + (col < n_cols ? col : 0);
     if constexpr (V % PER == 0) {
 #pragma unroll
@@ -655,12 +663,12 @@ __device__ __forceinline__ void st_vec_any(R* __restrict__ p, const VecT<R, V>& 
     *reinterpret_cast<u32x2_t*>(p) = __builtin_bit_cast(u32x2_t, v);
   }
 }
-template <typename R, int V, int NCH, bool FULL = false>
+template <typename R, int V, int NCH, bool FULL = false, int TPR = 256>
 __device__ __forceinline__ void load_row_any(const R* __restrict__ base, int n_cols,
                                              VecT<R, V> (&r)[NCH]) {
 #pragma unroll
   for (int k = 0; k < NCH; ++k) {
-    const int col = ((int)threadIdx.x + 256 * k) * V;
+    const int col = (row_tid<TPR>() + TPR * k) * V;
     r[k] = ld_vec_any<R, V>(base + ((FULL || col < n_cols) ? col : 0));
   }
 }
@@ -670,7 +678,7 @@ __device__ __forceinline__ void load_row_any(const R* __restrict__ base, int n_c
 // norm1, algebraic_model.py:150-151): h = x + r is rounded to T exactly as
 // torch's promoted add rounds it, written once, and normalised from registers,
 // so (h, y, mu) are bit-identical to the add followed by the plain norm.
-template <typename T, typename W, int NCH, typename R = void, typename Y = T, bool FULL = false>
+template <typename T, typename W, int NCH, typename R = void, typename Y = T, bool FULL = false, int TPR = 256>
 __global__ __launch_bounds__(256) void men_fwd_k(const T* __restrict__ x, const W* __restrict__ w,
                                                  Y* __restrict__ y, float* __restrict__ mu,
                                                  int64_t n_rows, int n_cols, int64_t ldx,
@@ -683,25 +691,26 @@ __global__ __launch_bounds__(256) void men_fwd_k(const T* __restrict__ x, const 
   const RT* r = reinterpret_cast<const RT*>(rp);
   __shared__ A red[2][kRowWaves];
   A wv[NCH][V];
-  load_weight<T, W, NCH>(w, n_cols, wv);
-  const int64_t G = gridDim.x;
-  int64_t row = blockIdx.x;
+  load_weight<T, W, NCH, TPR>(w, n_cols, wv);
+  constexpr int RPB = 256 / TPR;  // rows per block at a time
+  const int64_t G = (int64_t)gridDim.x * RPB;
+  int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / TPR;
   const int64_t last = n_rows - 1;
   VecT<T, V> cur[NCH], nx1[NCH];
   VecT<RT, V> rc[NCH], r1[NCH];
-  load_row<T, NCH, FULL>(x + std::min(row, last) * ldx, n_cols, cur);
-  if constexpr (kAdd) load_row_any<RT, V, NCH, FULL>(r + std::min(row, last) * ldr, n_cols, rc);
-  load_row<T, NCH, FULL>(x + std::min(row + G, last) * ldx, n_cols, nx1);
-  if constexpr (kAdd) load_row_any<RT, V, NCH, FULL>(r + std::min(row + G, last) * ldr, n_cols, r1);
+  load_row<T, NCH, FULL, TPR>(x + std::min(row, last) * ldx, n_cols, cur);
+  if constexpr (kAdd) load_row_any<RT, V, NCH, FULL, TPR>(r + std::min(row, last) * ldr, n_cols, rc);
+  load_row<T, NCH, FULL, TPR>(x + std::min(row + G, last) * ldx, n_cols, nx1);
+  if constexpr (kAdd) load_row_any<RT, V, NCH, FULL, TPR>(r + std::min(row + G, last) * ldr, n_cols, r1);
   for (int par = 0; row < n_rows; row += G, par ^= 1) {
     VecT<T, V> nx2[NCH];
     VecT<RT, V> r2[NCH];
-    load_row<T, NCH, FULL>(x + std::min(row + 2 * G, last) * ldx, n_cols, nx2);
+    load_row<T, NCH, FULL, TPR>(x + std::min(row + 2 * G, last) * ldx, n_cols, nx2);
     if constexpr (kAdd) {
-      load_row_any<RT, V, NCH, FULL>(r + std::min(row + 2 * G, last) * ldr, n_cols, r2);
+      load_row_any<RT, V, NCH, FULL, TPR>(r + std::min(row + 2 * G, last) * ldr, n_cols, r2);
 #pragma unroll
       for (int k = 0; k < NCH; ++k) {
-        const int col = ((int)threadIdx.x + 256 * k) * V;
+        const int col = (row_tid<TPR>() + TPR * k) * V;
 #pragma unroll
         for (int i = 0; i < V; ++i)
           cur[k].v[i] = from_acc<T>(to_acc(cur[k].v[i]) + to_acc(rc[k].v[i]));
@@ -711,17 +720,17 @@ __global__ __launch_bounds__(256) void men_fwd_k(const T* __restrict__ x, const 
     A s = A(0);
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
-      const bool in = chunk_in<FULL>(k, V, n_cols);
+      const bool in = chunk_in<FULL, TPR>(k, V, n_cols);
 #pragma unroll
       for (int i = 0; i < V; ++i) s += in ? fabs(to_acc(cur[k].v[i])) : A(0);  // fused_ops.py:324
     }
-    s = block_sum_par(s, red, par);
+    s = row_sum<TPR>(s, red, par);
     const A mean = s / A(n_cols);          // fused_ops.py:326
     const A inv = A(1) / (mean + A(eps));  // fused_ops.py:327
-    if (threadIdx.x == 0) mu[row] = (float)mean;  // fused_ops.py:330 (no eps)
+    if (row_tid<TPR>() == 0) mu[row] = (float)mean;  // fused_ops.py:330 (no eps)
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
-      const int col = ((int)threadIdx.x + 256 * k) * V;
+      const int col = (row_tid<TPR>() + TPR * k) * V;
       if (FULL || col < n_cols) {
         VecT<Y, V> o;
 #pragma unroll
@@ -751,7 +760,7 @@ constexpr int kNormPf = 2;
 // through the residual stream, and dx = round_T(norm_bwd) + dh (the sum
 // autograd forms for h, in T), written for x and, cast to R, for r (dr may
 // be null).
-template <typename T, typename W, int NCH, typename R = void, typename Y = T, bool FULL = false>
+template <typename T, typename W, int NCH, typename R = void, typename Y = T, bool FULL = false, int TPR = 256>
 __global__ __launch_bounds__(256) void men_bwd_k(
     const Y* __restrict__ dy, const T* __restrict__ x, const W* __restrict__ w,
     const float* __restrict__ mu, T* __restrict__ dx, typename AccT<T>::type* __restrict__ partial,
@@ -765,14 +774,15 @@ __global__ __launch_bounds__(256) void men_bwd_k(
   RT* dr = reinterpret_cast<RT*>(drp);
   __shared__ A red[2][kRowWaves];
   A wv[NCH][V], dg[NCH][V];
-  load_weight<T, W, NCH>(w, n_cols, wv);
+  load_weight<T, W, NCH, TPR>(w, n_cols, wv);
 #pragma unroll
   for (int k = 0; k < NCH; ++k)
 #pragma unroll
     for (int i = 0; i < V; ++i) dg[k][i] = A(0);
   const A e = A(eps);
-  const int64_t G = gridDim.x;
-  int64_t row = blockIdx.x;
+  constexpr int RPB = 256 / TPR;  // rows per block at a time
+  const int64_t G = (int64_t)gridDim.x * RPB;
+  int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / TPR;
   // ring of rows row, row + G, ..., row + PF*G: slot 0 is reduced next
   VecT<Y, V> by[PF + 1][NCH];
   VecT<T, V> bx[PF + 1][NCH], bh[PF + 1][NCH];
@@ -783,35 +793,35 @@ __global__ __launch_bounds__(256) void men_bwd_k(
 #pragma unroll
   for (int j = 0; j < PF; ++j) {
     const int64_t r = std::min(row + j * G, last);
-    load_row_any<Y, V, NCH, FULL>(dy + r * lddy, n_cols, by[j]);
-    load_row<T, NCH, FULL>(x + r * ldx, n_cols, bx[j]);
-    if constexpr (kAdd) load_row<T, NCH, FULL>(dh + r * lddh, n_cols, bh[j]);
+    load_row_any<Y, V, NCH, FULL, TPR>(dy + r * lddy, n_cols, by[j]);
+    load_row<T, NCH, FULL, TPR>(x + r * ldx, n_cols, bx[j]);
+    if constexpr (kAdd) load_row<T, NCH, FULL, TPR>(dh + r * lddh, n_cols, bh[j]);
     bm[j] = mu[r];  // the row statistic travels with its row
   }
   for (int par = 0; row < n_rows; row += G, par ^= 1) {
     {
       const int64_t r = std::min(row + PF * G, last);
-      load_row_any<Y, V, NCH, FULL>(dy + r * lddy, n_cols, by[PF]);
-      load_row<T, NCH, FULL>(x + r * ldx, n_cols, bx[PF]);
-      if constexpr (kAdd) load_row<T, NCH, FULL>(dh + r * lddh, n_cols, bh[PF]);
+      load_row_any<Y, V, NCH, FULL, TPR>(dy + r * lddy, n_cols, by[PF]);
+      load_row<T, NCH, FULL, TPR>(x + r * ldx, n_cols, bx[PF]);
+      if constexpr (kAdd) load_row<T, NCH, FULL, TPR>(dh + r * lddh, n_cols, bh[PF]);
       bm[PF] = mu[r];
     }
     const A inv = A(1) / ((A)bm[0] + e);  // fused_ops.py:389-390
     A cs = A(0);
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
-      const bool in = chunk_in<FULL>(k, V, n_cols);
+      const bool in = chunk_in<FULL, TPR>(k, V, n_cols);
 #pragma unroll
       for (int i = 0; i < V; ++i) {
         const A p = to_acc(bx[0][k].v[i]) * inv * wv[k][i];
         cs = in ? men_fma(to_acc(by[0][k].v[i]), p, cs) : cs;  // fused_ops.py:404-405
       }
     }
-    cs = block_sum_par(cs, red, par);
+    cs = row_sum<TPR>(cs, red, par);
     const A corr = cs / A(n_cols);  // fused_ops.py:408
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
-      const int col = ((int)threadIdx.x + 256 * k) * V;
+      const int col = (row_tid<TPR>() + TPR * k) * V;
       const bool in = FULL || col < n_cols;
       VecT<T, V> o;
 #pragma unroll
@@ -843,9 +853,29 @@ __global__ __launch_bounds__(256) void men_bwd_k(
       }
     }
   }
+  if constexpr (TPR != 256) {
+    // the block's waves hold partials of the same columns: wave 0 adds them in
+    // wave order, so that the launch still leaves one partial row per block
+    __shared__ A dsum[RPB - 1][NCH * V][TPR];
+    const int wv_ = threadIdx.x / TPR, t = row_tid<TPR>();
+    if (wv_ > 0) {
+#pragma unroll
+      for (int k = 0; k < NCH; ++k)
+#pragma unroll
+        for (int i = 0; i < V; ++i) dsum[wv_ - 1][k * V + i][t] = dg[k][i];
+    }
+    __syncthreads();
+    if (wv_ > 0) return;
+#pragma unroll
+    for (int j = 0; j < RPB - 1; ++j)
+#pragma unroll
+      for (int k = 0; k < NCH; ++k)
+#pragma unroll
+        for (int i = 0; i < V; ++i) dg[k][i] += dsum[j][k * V + i][t];
+  }
 #pragma unroll
   for (int k = 0; k < NCH; ++k) {
-    const int col = ((int)threadIdx.x + 256 * k) * V;
+    const int col = (row_tid<TPR>() + TPR * k) * V;
 #pragma unroll
     for (int i = 0; i < V; ++i)
       if (FULL || col + i < n_cols) partial[(int64_t)blockIdx.x * n_cols + col + i] = dg[k][i];
@@ -972,13 +1002,17 @@ template <typename A> __global__ void fill_zero_k(A* __restrict__ p, int64_t n) 
 // Host launchers
 // ============================================================================
 
-// Persistent row grids: up to `per_cu` 256-thread blocks per compute unit,
-// and at least 4 rows per block so the two-row prefetch (which clamps past
-// the last row) wastes little.
+// Persistent row grids: up to `per_cu` 256-thread blocks per compute unit. With
+// many rows a block takes at least 4, so that the two-row prefetch (which
+// clamps past the last row) wastes little; with few it takes 2 or 1, since the
+// rows of a block run one after the other (norm forward, one row per block
+// against 4: 8 x 4096 bf16 4.3 -> 2.3 us, 256 x 4096 5.4 -> 3.5, 512 x 2048
+// residual 7.4 -> 5.4; two: 2048 x 4096 11.3 -> 10.2; from 4096 rows on 4).
 constexpr int kRowBlocksPerCU = 8;
 static inline int64_t row_grid(int64_t rows, int per_cu) {
-  const int64_t cap = std::min<int64_t>((int64_t)per_cu * num_cus(), (rows + 3) / 4);
-  return std::max<int64_t>(1, std::min<int64_t>(rows, cap));
+  const int64_t cus = num_cus();
+  const int64_t per = rows <= 2 * cus ? 1 : rows <= 8 * cus ? 2 : 4;
+  return std::max<int64_t>(1, std::min<int64_t>((int64_t)per_cu * cus, (rows + per - 1) / per));
 }
 
 // grid of the one-block-per-row kernels, which walk rows with a grid stride
@@ -1024,6 +1058,39 @@ static inline bool kat_full_variant(int n, bool full) { return full && kat_full_
     case 4: { constexpr int N = 4; __VA_ARGS__; } break;  \
     case 8: { constexpr int N = 8; __VA_ARGS__; } break;  \
     default: { constexpr int N = 16; __VA_ARGS__; } break; \
+  }
+
+// Norm rows held by one wave (TPR = 64): chunk rounds of 64 16-byte chunks, 0
+// for the block-per-row kernels. Rows of up to 4 rounds (1024 fp32, 2048 16-bit
+// values) leave most of a 256-thread block idle and pay a barrier per row;
+// a wave per row needs no barrier and uses every lane. Measured, block / wave
+// (bf16): backward 32768 x 512 73 / 26 us, 16384 x 768 42.5 / 23.6, 16384 x 2048
+// 47.5 / 41.4, the residual norm of an fp32 stream 32768 x 768 76.9 / 69.9,
+// 16384 x 1024 51.8 / 48.6; forward 32768 x 512 26.6 / 16.5, 16384 x 768 17.1 /
+// 14.0, residual 32768 x 768 53.1 / 51.1, 16384 x 2048 27.6 / 27.9. Up to one
+// row per CU the block kernels are faster (one row each: 128 x 768 residual
+// backward 5.2 / 5.8 us).
+static inline int wave_norm_nch(int64_t rows, int64_t n_cols, int V) {
+  const int64_t need = (n_cols + 64 * V - 1) / (64 * V);
+  return rows > num_cus() && need <= 4 ? (int)need : 0;
+}
+// Forward blocks of 4 such rows: as many per CU as the registers of their two
+// prefetched rows keep resident (8 per CU: 16384 x 1024 residual 39.5 us
+// against 37.1 with 4, 4096 x 1024 fp32 11.0 against 8.8 with 2).
+static inline int64_t wave_row_grid(int64_t rows, int nchw) {
+  const int per_cu = nchw <= 2 ? 4 : nchw == 3 ? 3 : 2;
+  return std::min<int64_t>((rows + kRowWaves - 1) / kRowWaves, (int64_t)per_cu * num_cus());
+}
+#define KAT_NCHW_SWITCH(nch, full, ...)                                                           \
+  switch ((nch) * 2 + ((full) ? 1 : 0)) {                                                         \
+    case 2: { constexpr int N = 1; constexpr bool FULL = false; __VA_ARGS__; } break;             \
+    case 3: { constexpr int N = 1; constexpr bool FULL = true; __VA_ARGS__; } break;              \
+    case 4: { constexpr int N = 2; constexpr bool FULL = false; __VA_ARGS__; } break;             \
+    case 5: { constexpr int N = 2; constexpr bool FULL = true; __VA_ARGS__; } break;              \
+    case 6: { constexpr int N = 3; constexpr bool FULL = false; __VA_ARGS__; } break;             \
+    case 7: { constexpr int N = 3; constexpr bool FULL = true; __VA_ARGS__; } break;              \
+    case 8: { constexpr int N = 4; constexpr bool FULL = false; __VA_ARGS__; } break;             \
+    default: { constexpr int N = 4; constexpr bool FULL = true; __VA_ARGS__; } break;             \
   }
 
 template <typename T>
@@ -1148,7 +1215,14 @@ static int men_fwd_t(const T* x, const W* w, Y* y, float* mu, int64_t rows, int6
     vec = vec && ldr % V == 0 && ldh % V == 0 && aligned16(h) &&
           reinterpret_cast<uintptr_t>(r) % (V * sizeof(R)) == 0;
   const int nch = vec ? pick_nch(cols, 256 * V) : 0;
-  if (nch) {
+  const int nchw = vec ? wave_norm_nch(rows, cols, V) : 0;
+  if (nchw) {
+    const int64_t blocks = wave_row_grid(rows, nchw);
+    const bool full = cols == (int64_t)nchw * 64 * V;
+    KAT_NCHW_SWITCH(nchw, full, hipLaunchKernelGGL((men_fwd_k<T, W, N, R, Y, FULL, 64>), dim3((unsigned)blocks),
+                           dim3(256), 0, st, x, w, y, mu, rows, (int)cols, ldx, ldy, eps,
+                           (const void*)r, h, ldr, ldh));
+  } else if (nch) {
     const int64_t blocks = row_grid(rows, kRowBlocksPerCU);
     const bool full = cols == (int64_t)nch * 256 * V;
     KAT_NCH_SWITCH(nch, {
@@ -1168,11 +1242,19 @@ static int men_fwd_t(const T* x, const W* w, Y* y, float* mu, int64_t rows, int6
   return check_launch(kAdd ? "kat_add_men_fwd" : "kat_men_fwd");
 }
 
-// dgamma partials cost G x cols x 4 bytes of extra traffic (written here,
-// read by colsum_k): two blocks per CU.
-static int men_bwd_grid(int64_t rows, bool resident) {
-  (void)resident;
-  return (int)row_grid(rows, 2);
+// Backward blocks. The dgamma partials cost G x cols x 4 bytes of extra traffic
+// (written here, read by colsum_k), so G is two blocks per CU at most, one per
+// CU below 16 rows per CU (2048 x 2048 15.5 -> 12.9 us) and for waves that hold
+// 3 or 4 rounds of a row (16384 x 2048 46.4 -> 41.4; at 2 rounds, 16384 x 768,
+// one per CU is slower, 23.6 -> 30.0). Few rows: one or two per block, since a
+// block's rows run one after the other (8 x 768 7.2 -> 5.0, 512 x 2048
+// residual 10.6 -> 9.8). nchw: wave_norm_nch (0: a block per row).
+static int men_bwd_grid(int64_t rows, int nchw) {
+  const int64_t cus = num_cus();
+  if (nchw) return (int)std::min<int64_t>((rows + 2 * kRowWaves - 1) / (2 * kRowWaves), (nchw <= 2 ? 2 : 1) * cus);
+  if (2 * rows <= cus) return (int)std::max<int64_t>(1, rows);
+  if (rows <= 2 * cus) return (int)((rows + 1) / 2);
+  return (int)(rows < 16 * cus ? std::min<int64_t>((rows + 3) / 4, cus) : 2 * cus);
 }
 
 template <typename T, typename W, typename R = void, typename Y = T>
@@ -1192,12 +1274,18 @@ static int men_bwd_t(const Y* dy, const T* x, const W* w, const float* mu, T* dx
     vec = vec && lddh % V == 0 && aligned16(dh) &&
           (dr == nullptr || (lddr % V == 0 && reinterpret_cast<uintptr_t>(dr) % (V * sizeof(R)) == 0));
   const int nch = vec ? pick_nch(cols, 256 * V) : 0;
-  const int G = men_bwd_grid(rows, nch != 0);
+  const int nchw = vec ? wave_norm_nch(rows, cols, V) : 0;
+  const int G = men_bwd_grid(rows, nchw);
   const size_t need = (size_t)G * (size_t)cols * sizeof(A);
   if (ws_bytes < need || (need && ws == nullptr))
     return fail(KAT_EINVAL, "%s: workspace %zu bytes < required %zu", nm, ws_bytes, need);
   A* partial = reinterpret_cast<A*>(ws);
-  if (nch) {
+  if (nchw) {
+    const bool full = cols == (int64_t)nchw * 64 * V;
+    KAT_NCHW_SWITCH(nchw, full, hipLaunchKernelGGL((men_bwd_k<T, W, N, R, Y, FULL, 64>), dim3(G), dim3(256), 0, st,
+                           dy, x, w, mu, dx, partial, rows, (int)cols, lddy, ldx, lddx, eps, dh,
+                           lddh, (void*)dr, lddr));
+  } else if (nch) {
     const bool full = cols == (int64_t)nch * 256 * V;
     KAT_NCH_SWITCH(nch, {
       if (kat_full_variant(N, full))
@@ -1331,8 +1419,8 @@ extern "C" int kat_men_fwd(const void* x, const void* w, void* y, float* mu, int
 extern "C" size_t kat_men_bwd_workspace_size(int64_t n_rows, int64_t n_cols, int dtype) {
   const int sz = dtype_size(dtype);
   if (n_rows <= 0 || n_cols <= 0 || sz == 0) return 0;
-  // alignment decides between the two kernels at call time: size for the larger grid
-  const int G = std::max(men_bwd_grid(n_rows, true), men_bwd_grid(n_rows, false));
+  // alignment decides between the kernels at call time: size for the larger grid
+  const int G = std::max(men_bwd_grid(n_rows, 0), men_bwd_grid(n_rows, wave_norm_nch(n_rows, n_cols, 16 / sz)));
   const size_t acc = dtype == KAT_F64 ? 8 : 4;
   return (size_t)G * (size_t)n_cols * acc;
 }
