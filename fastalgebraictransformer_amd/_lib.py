@@ -84,6 +84,20 @@ def load():
     return _lib
 
 
+_ops = None
+
+
+def ops():
+    """The native autograd entry points (csrc/torch_ops.cpp, linked to
+    libkat.so), imported once; raise if they are not built."""
+    global _ops
+    if _ops is None:
+        load()
+        from . import _katops
+        _ops = _katops
+    return _ops
+
+
 def dtype_code(t):
     try:
         return _DTYPES[t.dtype]

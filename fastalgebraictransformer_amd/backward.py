@@ -7,6 +7,8 @@ Same Python API as the reference ``kernels.backward``
 (backward.py:7-46): with p = f / (L + eps) and g = 2 / ((|s|+1)^2 (sigma+eps)),
 dS = p g (dO.v - Delta), dq = scale dS K, dk = scale dS^T Q, dv = P^T dO.
 The launch goes to ``kat_attn_bwd`` in libkat.so (deterministic: no atomics).
+The functional wrappers run the native autograd functions of csrc/torch_ops.cpp
+and, for what those do not take (they return None), the classes here.
 """
 
 import torch
@@ -101,7 +103,8 @@ class RationalAttentionFunction(torch.autograd.Function):
 
 def rational_attention(q, k, v, alibi_slopes, scale, causal=True, eps=EPS):
     """Causal ALiBi rational attention with a recompute backward."""
-    return RationalAttentionFunction.apply(q, k, v, alibi_slopes, scale, causal, eps)
+    o = _lib.ops().attention(q, k, v, alibi_slopes, scale, eps) if q.is_cuda else None
+    return RationalAttentionFunction.apply(q, k, v, alibi_slopes, scale, causal, eps) if o is None else o
 
 
 class PackedRationalAttention(torch.autograd.Function):
@@ -146,7 +149,8 @@ def rational_attention_packed(qkv, alibi_slopes, scale, eps=EPS, key_mask=None):
     """Causal ALiBi rational attention on qkv [B, T, 3, H, D]; returns
     [B, T, H, D] (see PackedRationalAttention). ``key_mask`` [B, T]: keys where
     it is 0 are dropped (see rational_attention_masked)."""
-    return PackedRationalAttention.apply(qkv, alibi_slopes, scale, eps, key_mask)
+    y = _lib.ops().attention_packed(qkv, alibi_slopes, scale, eps, key_mask) if qkv.is_cuda else None
+    return PackedRationalAttention.apply(qkv, alibi_slopes, scale, eps, key_mask) if y is None else y
 
 
 class MaskedRationalAttentionFunction(torch.autograd.Function):
@@ -212,6 +216,9 @@ def rational_attention_masked(q, k, v, alibi_slopes, scale, key_mask=None, causa
     CUDA tensors run the libkat kernels; CPU tensors the reference's torch
     formulation (attention_torch)."""
     if q.is_cuda:
+        o = _lib.ops().attention_masked(q, k, v, alibi_slopes, scale, key_mask, bool(causal), eps)
+        if o is not None:
+            return o
         return MaskedRationalAttentionFunction.apply(q, k, v, alibi_slopes, scale, key_mask,
                                                      causal, eps)
     return attention_torch(q, k, v, alibi_slopes, scale, key_mask, causal, eps)

@@ -185,6 +185,9 @@ def rational_attention_decode(q, k_cache, v_cache, alibi_slopes, scale, lengths=
     B, H, D = q.shape
     T = k_cache.shape[2]
     assert tuple(k_cache.shape) == (B, H, T, D) and tuple(v_cache.shape) == (B, H, T, D)
+    r = _lib.ops().decode(q, k_cache, v_cache, alibi_slopes, scale, lengths, eps)
+    if r is not None:
+        return r
     lib = _lib.load()
     k_cache, v_cache = k_cache.to(q.dtype), v_cache.to(q.dtype)
     q, k_cache, v_cache = _unit_d(q), _unit_d(k_cache), _unit_d(v_cache)

@@ -4,7 +4,10 @@ Same Python API as the reference ``kernels.fused_ops``
 (SkyeGunasekaran/fastAlgebraicTransformer, fused_ops.py:20-21 constants,
 :435-599 autograd Functions, :606-636 functional wrappers). CUDA (HIP) tensors
 run the hand-written gfx950 kernels of libkat.so through its C ABI; there is no
-other GPU path. CPU tensors keep the reference's own torch formulas
+other GPU path. The functional wrappers run the native autograd functions of
+csrc/torch_ops.cpp; what those do not take (they return None: subclasses,
+transforms, tracing, mixed dtypes, empty or wrongly shaped inputs) runs the
+torch.autograd.Function classes below, the same kernels. CPU tensors keep the reference's own torch formulas
 (fused_ops.py:610-615, 623-626, 634-636), as the reference does.
 
 Differences from the reference launch wrappers, all layout-only:
@@ -258,7 +261,8 @@ class ResidualMeanErrorNorm(torch.autograd.Function):
 def rational_softmax(x, eps=EPS):
     """Rational softmax over the last dim (reference fused_ops.py:606-615)."""
     if x.is_cuda:
-        return RationalSoftmax.apply(x, eps)
+        p = _lib.ops().softmax(x, eps)
+        return RationalSoftmax.apply(x, eps) if p is None else p
     sig = 0.5 * (x / (x.abs() + 1.0) + 1.0)
     f = sig.pow(4)
     return f / (f.sum(dim=-1, keepdim=True) + eps)
@@ -267,7 +271,8 @@ def rational_softmax(x, eps=EPS):
 def rational_swiglu(gate, value):
     """gate * sigma(gate) * value (reference fused_ops.py:618-626)."""
     if gate.is_cuda:
-        return RationalSwiGLU.apply(gate, value)
+        y = _lib.ops().swiglu(gate, value)
+        return RationalSwiGLU.apply(gate, value) if y is None else y
     sig = 0.5 * (gate / (gate.abs() + 1.0) + 1.0)
     return gate * sig * value
 
@@ -275,7 +280,8 @@ def rational_swiglu(gate, value):
 def mean_error_norm(x, weight, eps=EPS):
     """x / (mean|x| + eps) * weight (reference fused_ops.py:629-636)."""
     if x.is_cuda:
-        return MeanErrorNorm.apply(x, weight, eps)
+        y = _lib.ops().norm(x, weight, eps)
+        return MeanErrorNorm.apply(x, weight, eps) if y is None else y
     m = x.abs().mean(dim=-1, keepdim=True)
     return (x / (m + eps)) * weight
 
@@ -288,7 +294,8 @@ def add_mean_error_norm(x, r, weight, eps=EPS, out_dtype=None):
     if out_dtype == x.dtype:
         out_dtype = None
     if x.is_cuda:
-        return ResidualMeanErrorNorm.apply(x, r, weight, eps, out_dtype)
+        hy = _lib.ops().add_norm(x, r, weight, eps, out_dtype)
+        return ResidualMeanErrorNorm.apply(x, r, weight, eps, out_dtype) if hy is None else hy
     h = x + r
     y = mean_error_norm(h, weight, eps)
     return h, (y if out_dtype is None else y.to(out_dtype))
@@ -298,6 +305,7 @@ def rational_swiglu_packed(gv):
     """gate * sigma(gate) * value with gate, value = gv.chunk(2, dim=-1)
     (see PackedRationalSwiGLU); CPU tensors use the reference formula."""
     if gv.is_cuda:
-        return PackedRationalSwiGLU.apply(gv)
+        y = _lib.ops().swiglu_packed(gv)
+        return PackedRationalSwiGLU.apply(gv) if y is None else y
     gate, value = gv.chunk(2, dim=-1)
     return rational_swiglu(gate, value)
