@@ -300,11 +300,23 @@ template <typename A> __device__ __forceinline__ A block_sum_par(A v, A (*red)[k
   return (red[par][0] + red[par][1]) + (red[par][2] + red[par][3]);
 }
 
-// Sum over a row's threads: the block's 256, or one wave's 64 (no barrier)
+// Sum over a row's threads: the block's 256, or one wave's 64 (no barrier). The
+// wave's last two steps add in fp64: they carry the row's whole magnitude, and
+// their rounding would set the error of narrow fp32 rows (768 columns: 6.9e-8
+// of y against 6.6e-8 for a block's sum, 6.5e-8 this way).
 template <int TPR, typename A> __device__ __forceinline__ A row_sum(A v, A (*red)[kRowWaves], int par) {
   if constexpr (TPR == 256) return block_sum_par(v, red, par);
-  else return wave_sum(v);
+#pragma unroll
+  for (int off = 32; off > 2; off >>= 1) v += __shfl_xor(v, off, 64);
+  double d = (double)v;
+  d += __shfl_xor(d, 2, 64);
+  d += __shfl_xor(d, 1, 64);
+  return (A)d;
 }
+
+template <typename A> __device__ __forceinline__ A pair_sum(const A (&a)[1]) { return a[0]; }
+template <typename A> __device__ __forceinline__ A pair_sum(const A (&a)[2]) { return a[0] + a[1]; }
+template <typename A> __device__ __forceinline__ A pair_sum(const A (&a)[4]) { return (a[0] + a[1]) + (a[2] + a[3]); }
 
 // Loads this thread's chunks of one row. Chunks past the row end re-read the
 // row's first chunk (always in bounds) and are masked where they are used:
@@ -717,14 +729,17 @@ __global__ __launch_bounds__(256) void men_fwd_k(const T* __restrict__ x, const 
         if (FULL || col < n_cols) st_vec<T, V>(h + row * ldh + col, cur[k]);
       }
     }
-    A s = A(0);
+    // NA running sums: a wave's lane sums four times the elements of a block's
+    // thread, in chains of the same length
+    constexpr int NA = TPR == 256 ? 1 : V < 4 ? V : 4;
+    A sa[NA] = {};
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
       const bool in = chunk_in<FULL, TPR>(k, V, n_cols);
 #pragma unroll
-      for (int i = 0; i < V; ++i) s += in ? fabs(to_acc(cur[k].v[i])) : A(0);  // fused_ops.py:324
+      for (int i = 0; i < V; ++i) sa[i % NA] += in ? fabs(to_acc(cur[k].v[i])) : A(0);  // fused_ops.py:324
     }
-    s = row_sum<TPR>(s, red, par);
+    A s = row_sum<TPR>(pair_sum(sa), red, par);
     const A mean = s / A(n_cols);          // fused_ops.py:326
     const A inv = A(1) / (mean + A(eps));  // fused_ops.py:327
     if (row_tid<TPR>() == 0) mu[row] = (float)mean;  // fused_ops.py:330 (no eps)
@@ -807,17 +822,18 @@ __global__ __launch_bounds__(256) void men_bwd_k(
       bm[PF] = mu[r];
     }
     const A inv = A(1) / ((A)bm[0] + e);  // fused_ops.py:389-390
-    A cs = A(0);
+    constexpr int NA = TPR == 256 ? 1 : V < 4 ? V : 4;  // as in men_fwd_k
+    A ca[NA] = {};
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
       const bool in = chunk_in<FULL, TPR>(k, V, n_cols);
 #pragma unroll
       for (int i = 0; i < V; ++i) {
         const A p = to_acc(bx[0][k].v[i]) * inv * wv[k][i];
-        cs = in ? men_fma(to_acc(by[0][k].v[i]), p, cs) : cs;  // fused_ops.py:404-405
+        ca[i % NA] = in ? men_fma(to_acc(by[0][k].v[i]), p, ca[i % NA]) : ca[i % NA];  // fused_ops.py:404-405
       }
     }
-    cs = row_sum<TPR>(cs, red, par);
+    const A cs = row_sum<TPR>(pair_sum(ca), red, par);
     const A corr = cs / A(n_cols);  // fused_ops.py:408
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
@@ -958,8 +974,8 @@ __global__ __launch_bounds__(256) void men_bwd_mp_k(
 
 // dw[c] = sum_g partial[g][c] in a fixed order. A block owns 16 columns and
 // 64 row groups (4 per wave, 16 waves): row group rg adds rows rg, rg + 64, ...
-// in two interleaved accumulators, then the 64 group sums are added in group
-// order. 16 columns per block give cols / 16 blocks (256 at 4096 columns), so
+// in two interleaved accumulators, then the 64 group sums are added in eight
+// chains of eight and those pairwise (fixed order). 16 columns per block give cols / 16 blocks (256 at 4096 columns), so
 // the reduction spreads over the whole chip.
 // 16 fp32 columns are half a 128-byte line: the two blocks that share a line
 // are blocks b and b + 8, which the dispatcher places on the same XCD (blocks
@@ -986,10 +1002,10 @@ __global__ __launch_bounds__(1024) void colsum_k(const A* __restrict__ partial, 
   red[rg][c] = s0 + s1;
   __syncthreads();
   if (threadIdx.x < 16 && cg * 16 + (int)threadIdx.x < n_cols) {
-    A t = A(0);
-#pragma unroll 8
-    for (int i = 0; i < 64; ++i) t += red[i][threadIdx.x];
-    out[cg * 16 + threadIdx.x] = t;
+    A t[8] = {};
+#pragma unroll
+    for (int i = 0; i < 64; ++i) t[i & 7] += red[i][threadIdx.x];
+    out[cg * 16 + threadIdx.x] = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
   }
 }
 
