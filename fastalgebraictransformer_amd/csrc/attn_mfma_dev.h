@@ -274,20 +274,19 @@ template <int D, int NW, int ROWS = 64> struct TileDma {
 };
 
 // Block order. Workgroups are dispatched round-robin over the 8 XCDs (block id
-// i runs on XCD i % 8), and each XCD has its own L2. Heads are assigned to XCDs
-// (head h on XCD h % 8 when B*H is a multiple of 8) and each XCD takes the
-// tiles of its heads longest (most causal work) first across all its heads,
-// which balances the causal triangle over the XCD's CUs.
+// i runs on XCD i % 8), and each XCD has its own L2. The XCDs form g = gcd(B*H, 8)
+// classes (XCD x in class x % g) and head h's blocks run in class h % g: on one
+// XCD when B*H is a multiple of 8, on two when it is 4 modulo 8. Each class
+// takes the tiles of its heads longest (most causal work) first across all
+// its heads, which balances the causal triangle over its CUs.
 // Returns the (b*H + h) index and the tile rank (0 = most work).
 __device__ __forceinline__ void block_order(int id, int BH, int& bh, int& rank) {
-  if ((BH & 7) == 0) {
-    const int xcd = id & 7, slot = id >> 3, hpx = BH >> 3;
-    rank = slot / hpx;
-    bh = xcd + 8 * (slot - rank * hpx);
-  } else {
-    rank = id / BH;
-    bh = id - rank * BH;
-  }
+  const int lg = (BH & 7) == 0 ? 3 : (BH & 3) == 0 ? 2 : (BH & 1) == 0 ? 1 : 0;  // log2 g
+  const int cls = id & ((1 << lg) - 1);
+  const int pos = id >> lg;  // the block's place in its class: (slot, XCD of the class)
+  const int hpc = BH >> lg;  // heads per class
+  rank = pos / hpc;
+  bh = cls + ((pos - rank * hpc) << lg);
 }
 
 // Epilogue staging: a wave's output rows (R rows of D 16-bit elements) pass

@@ -19,7 +19,7 @@
 //
 // Common structure of the forward and dK/dV kernels (the dQ kernel is a plain
 // streaming GEMM, described at it). Each wave owns 32 rows (queries, or keys
-// for dK/dV; 16 or 64 keys at some head dims, see dkv_keys) whose
+// for dK/dV; 16 keys at D = 256 and for small grids, see dkv_keys) whose
 // operand fragments stay in VGPRs as the B operand of v_mfma_f32_16x16x32; the
 // streamed side is staged 64 rows at a time by LDS-DMA into a swizzled,
 // double-buffered LDS tile and read as the A operand, either row-wise
@@ -693,22 +693,21 @@ constexpr int kDqS = 4;             // stages (32 keys each)
 // 64 queries would take all 256 VGPRs) a 32-query half of one; a block covers
 // kDqW waves' queries, i.e. a whole dS run (kQB tiles) or half of one
 template <int D> constexpr int dq_qw() { return D == 256 ? 32 : 64; }
-template <int D> constexpr int dq_block_queries() { return kDqW * dq_qw<D>(); }
 
-template <int D> struct DqSmem {
-  short k[kDqS][32 * D];                   // K rows (converted in place to K16)
-  short s[kDqS][kDqW][32 * dq_qw<D>()];    // each wave's dS^T rows
+template <int D, int QW> struct DqSmem {
+  short k[kDqS][32 * D];           // K rows (converted in place to K16)
+  short s[kDqS][kDqW][32 * QW];    // each wave's dS^T rows
 };
 
-template <typename T, int D, int MODE, int DE = D>
+template <typename T, int D, int MODE, int DE = D, int QW = dq_qw<D>()>
 __global__ __launch_bounds__(64 * kDqW, 1) void attn_bwd_dq_k(AttnArgs a, const int* __restrict__ kexp,
                                                               const int* __restrict__ ktile,
                                                               const f16* __restrict__ dst, int bh0, int G,
                                                               int kb0, int nk, float* __restrict__ dqacc) {
   typedef Mfma<T> M;
   constexpr int DS = DE / 16;
-  constexpr int QW = dq_qw<D>(), QC = QW / 16;  // queries per wave, 16-query column groups
-  constexpr int BQ = dq_block_queries<D>();      // queries per block
+  constexpr int QC = QW / 16;      // 16-query column groups
+  constexpr int BQ = kDqW * QW;    // queries per block
   constexpr int WPT = 64 / QW;                   // waves per 64-query tile
   constexpr bool kCausal = (MODE & kModeCausal) != 0;
   // K16 rows: 1 KB DMA segments over the first KW waves (all 8 at D = 128,
@@ -716,7 +715,7 @@ __global__ __launch_bounds__(64 * kDqW, 1) void attn_bwd_dq_k(AttnArgs a, const 
   constexpr int KW = std::min(kDqW, 32 * D / 512);
   typedef TileDma<D, KW, 32> KDma;
   typedef TileDma<QW, 1, 32> SDma;
-  __shared__ DqSmem<D> sm;
+  __shared__ DqSmem<D, QW> sm;
 
   const int T_ = a.T, H = a.H;
   const int n_qb = (T_ + BQ - 1) / BQ;
@@ -913,28 +912,33 @@ __global__ __launch_bounds__(64 * kDqW, 1) void attn_bwd_dq_k(AttnArgs a, const 
 // through LDS; a tile is worked in two 32-query chunks with one barrier each:
 //   phase 1: P role S, P, w of chunk c                    | barrier
 //   phase 2: P role dV(c); D role dP(c + 1), dS(c), dK(c)
-// The D role computes dP one chunk ahead (KR = 32) so that the reads of w
+// At D = 32 and 128 the D role computes dP one chunk ahead so that the reads of w
 // issued after the barrier overlap with MFMAs.
 // ============================================================================
 template <int D, int KS>
 struct DkvSmem {
   short q[2][kBN * D];         // Q16 tiles
   short o[2][kBN * D];         // dO tiles
-  f32x4 x[2][kNW][2 * KS][64];  // w: [chunk parity][key group][16-query half x ks][lane]
+  // the stats before w: at D = 64 every stats address then lies within the
+  // 64 KB immediate of an LDS read
   float st[2][2 * kBN];        // the tile's stats: 4 cinv of its queries, then -4 cinv Delta
   float km[kNW];               // KS = 1: the key groups' max |k| (pairs share an exponent)
+  f32x4 x[2][kNW][2 * KS][64];  // w: [chunk parity][key group][16-query half x ks][lane]
 };
 
-// KR: keys per wave pair. 32 at D = 32 and 128; 64 at D = 64 (twice the
-// MFMAs per LDS read of the streamed Q16 / dO tiles, in the registers D = 128
-// takes for 32 keys: backward 9-10% faster than 32 keys; at D = 32, whose
-// time is the per-score VALU work, 64 keys measured 10-13% slower); 16 at
-// D = 256 (whose B fragments and accumulators of 32 keys would exceed the
-// register budget), the two pairs of a 32-key group then sharing one K16
-// exponent. K16 exponents are per 32 keys at every KR.
-template <int D> constexpr int dkv_keys() { return D == 256 ? 16 : D == 64 ? 64 : kRows; }
+// KR: keys per wave pair: 32 at D <= 128, 16 at D = 256 (whose B fragments and
+// accumulators of 32 keys would exceed the register budget) and for small
+// grids (bwd_small_dkv); the two pairs of a 32-key group then share one K16
+// exponent (K16 exponents are per 32 keys at every KR). At D = 64 the kernel is
+// held to 128 registers, so that two blocks (four waves per SIMD) run per CU:
+// 64 keys per wave pair, one block per CU, reads each LDS fragment for
+// twice the MFMAs but issues MFMA, VALU and LDS work from two waves per SIMD
+// only (backward, bf16: B=16, H=12, T=2048 578 against 559 us, B=4, H=32,
+// T=4096 1366 against 1272, B=32, H=12, T=512 143 against 125, non-causal
+// 4 x 12 x 2048 302 against 275; bit-identical in causal mode).
+template <int D> constexpr int dkv_keys() { return D == 256 ? 16 : kRows; }
 template <typename T, int D, int MODE, int KR = kRows, int DE = D>
-__global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float* __restrict__ stats,
+__global__ __launch_bounds__(512, D == 64 && KR == 32 ? 4 : 1) void attn_bwd_dkv_k(AttnArgs a, const float* __restrict__ stats,
                                                          const f16* __restrict__ q16,
                                                          const int* __restrict__ qexp,
                                                          const int* __restrict__ ktile,
@@ -947,7 +951,6 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
   constexpr bool kCausal = (MODE & kModeCausal) != 0;
   constexpr bool kKM = (MODE & kModeKeyMask) != 0;
   constexpr int KS = KR / 16;     // 16-key groups per wave
-  constexpr int NE = (KS + 1) / 2;  // K16 exponents per wave (one per 32 keys; 16-key group ks takes ks / 2)
   constexpr int BK = kNW * KR;    // keys per block
   __shared__ DkvSmem<D, KS> sm;
 
@@ -1001,18 +1004,13 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
 
   // B operands: K16^T (P role) or V^T (D role) fragments; lane (g, li) holds row
   // kw + 16 ks + li, columns 32 kk + 8 g .. +7
-  // (P role: scaled by 2^ekw[ks / 2], the exponent tile_exp gives their 32 keys)
+  // (P role: scaled by 2^ekw, the exponent tile_exp gives their 32 keys)
   i16x8 bfr[KS][KK];
-  int ekw[NE];
+  int ekw = 0;
   {
     const __amdgpu_buffer_rsrc_t rk = rsrc(kp, row_bytes(T_, sk2, DR));
     const __amdgpu_buffer_rsrc_t rv = rsrc(vp, row_bytes(T_, sv2, DR));
-    float km[NE];
-#pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      km[e] = 0.f;
-      ekw[e] = 0;
-    }
+    float km = 0.f;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const uint32_t key = (uint32_t)(kw + 16 * ks + li);
@@ -1021,7 +1019,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
         const int col = 32 * kk + 8 * g;
         if (prole) {
           bfr[ks][kk] = load16(rk, col_off((key * sk2 + col) * 2, col, DR));
-          km[ks / 2] = fmaxf(km[ks / 2], absmax8<T>(bfr[ks][kk]));
+          km = fmaxf(km, absmax8<T>(bfr[ks][kk]));
         } else {
           bfr[ks][kk] = load16(rv, col_off((key * sv2 + col) * 2, col, DR));
         }
@@ -1029,31 +1027,24 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
     }
     if (prole) {
 #pragma unroll
-      for (int e = 0; e < NE; ++e)
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) km[e] = fmaxf(km[e], __shfl_xor(km[e], o, 64));
+      for (int o = 32; o > 0; o >>= 1) km = fmaxf(km, __shfl_xor(km, o, 64));
     }
     if constexpr (KS == 1) {
       // the 32-key group's two 16-key halves (waves grp and grp ^ 1) share one
       // exponent: the max of both
-      if (prole && lane == 0) sm.km[grp] = km[0];
+      if (prole && lane == 0) sm.km[grp] = km;
       __syncthreads();
-      if (prole) km[0] = fmaxf(km[0], sm.km[grp ^ 1]);
+      if (prole) km = fmaxf(km, sm.km[grp ^ 1]);
     }
     if (prole) {
+      ekw = tile_exp(km);
+      // the dQ kernel converts these 32 keys with the same exponent
+      if (lane == 0 && kw < T_ && (KS >= 2 || (grp & 1) == 0)) kexp[(int64_t)bh * ((T_ + 31) / 32) + (kw >> 5)] = ekw;
+      const float fk = ldexpf(1.f, ekw);
 #pragma unroll
-      for (int e = 0; e < NE; ++e) {
-        ekw[e] = tile_exp(km[e]);
-        // the dQ kernel converts these 32 keys with the same exponent
-        if (lane == 0 && kw + 32 * e < T_ && (KS >= 2 || (grp & 1) == 0))
-          kexp[(int64_t)bh * ((T_ + 31) / 32) + (kw >> 5) + e] = ekw[e];
-      }
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const float fk = ldexpf(1.f, ekw[ks / 2]);
+      for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) bfr[ks][kk] = to_f16x8s<T>(bfr[ks][kk], fk);
-      }
     }
   }
   // S layout: lane (g, li) element j holds q = qh + 4 g + j, key = kw + 16 ks + li
@@ -1063,18 +1054,12 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
   // bias in use (negated for query chunks wholly below this wave's keys in
   // non-causal mode). S comes out of the MFMA scaled by 2^(eq + ekw) (eq: the
   // Q16 tile's exponent): cbx carries that factor and sc = scale 2^-(eq + ekw)
-  // removes it (one of each per K16 exponent); the dK accumulators hold
+  // removes it; the dK accumulators hold
   // 2^(eq + kq) times the sum (kq: the query tile's dS exponent), rescaled
   // when a tile brings other exponents.
   int eq = 0, kq = 0;
-  float sfac[NE], sc[NE];  // 2^(eq + ekw), scale 2^-(eq + ekw)
-  f32x4 cbx[NE];
-#pragma unroll
-  for (int e = 0; e < NE; ++e) {
-    sfac[e] = ldexpf(1.f, ekw[e]);
-    cbx[e] = cb * sfac[e];
-    sc[e] = ldexpf(scale, -ekw[e]);
-  }
+  float sfac = ldexpf(1.f, ekw), sc = ldexpf(scale, -ekw);  // 2^(eq + ekw), scale 2^-(eq + ekw)
+  f32x4 cbx = cb * sfac;
   float slx = slope;
   // Padding mask: a dropped key's P and dS column is zero, so its dK / dV
   // rows are zero and the other keys' rows do not depend on it. The kernel
@@ -1125,7 +1110,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
   auto m1 = [&](auto role, int hr, f32x4 (&s_)[KS], const short* as_) __attribute__((always_inline)) {
     constexpr bool P = decltype(role)::value;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) s_[ks] = P ? cbx[ks / 2] : f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int ks = 0; ks < KS; ++ks) s_[ks] = P ? cbx : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
       const i16x8 fa = lds16(as_ + soff<D>(hr + li, 32 * kk + 8 * g));
@@ -1150,7 +1135,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
       f32x4 wv;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        float s = fmaf(s_[ks][j], sc[ks / 2], tterm);
+        float s = fmaf(s_[ks][j], sc, tterm);
         if constexpr (DIAG && !kCausal) {
           const int dkq = (kw + 16 * ks + li) - (qh + 4 * g + j);
           if (dkq > 0) s = fmaf(-2.f * slope, (float)dkq, s);
@@ -1216,12 +1201,13 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
   if (n_it > 0) issue(0, qbase);
   if (prole) dma_wait();
   __syncthreads();
-  // D role: dP of the current and the next chunk (KS = 2). At KS = 4 the
-  // registers of the next chunk's dP do not fit beside the rest, and at KS = 1
-  // (D = 256) they cost spills in the non-causal modes: dP is then computed in
-  // its own step, after the barrier (its MFMAs cover the reads of w; D = 256
-  // measured 0-3% faster causal and 8% non-causal, bit-identical)
-  constexpr bool kAhead = KS == 2;
+  // D role: dP of the current and the next chunk. Computed ahead only where one
+  // block's two waves per SIMD run alone and the registers are there (D = 32 and
+  // 128, 32 keys per wave): with two blocks per CU (D = 64, 128 registers) the
+  // look-ahead would spill, and at 16 keys per wave it does in the
+  // non-causal modes (D = 256 measured 0-3% faster causal and 8% non-causal
+  // without, bit-identical); dP is then computed after the barrier, half by half
+  constexpr bool kAhead = KS == 2 && D != 64;
   f32x4 dpA[2][KS], dpB[2][KS];
   if (kAhead && !prole && needc(0)) {
     m1(std::false_type{}, 0, dpA[0], sm.o[0]);
@@ -1244,12 +1230,9 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
       const int eqt = qexp_h[(qbase >> 6) + it], kqt = ktile_h[(qbase >> 6) + it];
       if (eqt != eq) {
         const float f = ldexpf(1.f, eqt - eq);
-#pragma unroll
-        for (int e = 0; e < NE; ++e) {
-          sfac[e] *= f;
-          sc[e] = ldexpf(sc[e], eq - eqt);
-          if constexpr (kCausal) cbx[e] *= f;
-        }
+        sfac *= f;
+        sc = ldexpf(sc, eq - eqt);
+        if constexpr (kCausal) cbx *= f;
       }
       p4 = ldexpf(0.25f, -kqt);
       // D role: this query tile's dS^T tile (both of its chunks)
@@ -1266,8 +1249,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
     }
     if constexpr (!kCausal) {
       const bool above = kw > qc + 31;
-#pragma unroll
-      for (int e = 0; e < NE; ++e) cbx[e] = (above ? -cb : cb) * sfac[e];
+      cbx = (above ? -cb : cb) * sfac;
       slx = above ? -slope : slope;
     }
     if (prole && need) {
@@ -1297,7 +1279,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
       // w of this chunk (read whether or not the chunk is needed: the buffer
       // always exists, and a conditional read leaves the compiler zeroing the
       // registers on the other path every chunk)
-      // (KS = 4: each half's w just before its use)
+      // (without look-ahead: each half's w just before its use)
       f32x4 wv[2 * KS];
       if constexpr (kAhead) {
 #pragma unroll
@@ -1310,9 +1292,6 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
           m1(std::false_type{}, r1, pnext[0], os1);
           m1(std::false_type{}, r1 + 16, pnext[1], os1);
         }
-      } else if (need) {
-        m1(std::false_type{}, r0, pcur[0], sm.o[buf]);
-        m1(std::false_type{}, r0 + 16, pcur[1], sm.o[buf]);
       }
       if (need) {
 #pragma unroll
@@ -1321,6 +1300,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
           const f32x4 ndv = *reinterpret_cast<const f32x4*>(sm.st[buf] + kBN + r0 + 16 * hh + 4 * g);
           uint32_t (&dp)[KS][2] = hh ? pb : pa;
           if constexpr (!kAhead) {
+            m1(std::false_type{}, r0 + 16 * hh, pcur[hh], sm.o[buf]);
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) wv[KS * hh + ks] = xw[KS * hh + ks][lane];
           }
@@ -1377,12 +1357,11 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkv_k(AttnArgs a, const float
   const int64_t ostr = prole ? a.sdv[2] : a.sdk[2];
   const float osc = prole ? 1.f : ldexpf(scale, -(kq + eq));  // dK: dS's 2^kq and Q16's 2^eq undone (exact)
   // the wave's KR rows (keys) through its own KR x D staging tile in the now
-  // idle tile and exchange buffers (8 waves x KR x D x 2 bytes within the
-  // Q16, dO and w buffers)
+  // idle tile buffers (8 waves x KR x D x 2 bytes within the Q16 and dO tiles)
   typedef DkvSmem<D, KS> Smem;
-  static_assert(sizeof(sm.q) + sizeof(sm.o) + sizeof(sm.x) >= 8 * KR * D * 2 && offsetof(Smem, q) == 0 &&
-                    offsetof(Smem, o) == sizeof(sm.q) && offsetof(Smem, x) == sizeof(sm.q) + sizeof(sm.o),
-                "staging tiles fit the tile and exchange buffers");
+  static_assert(sizeof(sm.q) + sizeof(sm.o) >= 8 * KR * D * 2 && offsetof(Smem, q) == 0 &&
+                    offsetof(Smem, o) == sizeof(sm.q),
+                "staging tiles fit the tile buffers");
   short* const et = reinterpret_cast<short*>(&sm) + w * KR * D;
   __syncthreads();  // every wave is done with the tile buffers
 #pragma unroll
@@ -1423,8 +1402,9 @@ inline int mfma_eff(int64_t D) {
 // the dS^T tiles, and (banded calls only) one head's fp32 dQ partial sums.
 // The dS^T region holds ds_cap() bytes of the call's mode's tiles (causal: the
 // lower triangle of each head's 64 x 64 tiles, ~T^2 bytes per head; non-causal:
-// all, ~2 T^2 bytes): as many heads as fit (a multiple of 8 when there are 8 or
-// more, so that heads keep their XCD), and dK/dV + dQ run per group of heads.
+// all, ~2 T^2 bytes): every head when they fit, else as many as do (a multiple of
+// 8 when there are 8 or more, so that heads keep their XCD), and dK/dV + dQ
+// run per group of heads.
 // When one head's tiles exceed the cap, the head's key tiles split into bands
 // of kQB-tile multiples (the widest whose first band fits the cap, at least
 // kQB tiles = 512 keys) and dK/dV + dQ run per band of each head, dQ
@@ -1450,7 +1430,7 @@ inline BwdWs bwd_ws(void* base, int64_t B, int64_t H, int64_t T, int64_t D, bool
   size_t ds_bytes, acc_bytes = 0;
   if (head <= cap) {
     group = std::max<int64_t>(1, std::min<int64_t>(BH, (int64_t)(cap / head)));
-    if (group >= 8) group &= ~(int64_t)7;
+    if (group < BH && group >= 8) group &= ~(int64_t)7;
     ds_bytes = (size_t)group * head;
   } else {
     // the widest band (a multiple of kQB key tiles) whose tiles fit the cap;
@@ -1526,6 +1506,60 @@ template <typename T, int D, int DE, int MODE> int launch_fwd(const AttnArgs& a,
   return check_launch("kat_attn_fwd (mfma)");
 }
 
+// Small grids. A dK/dV block is one per CU and walks every query chunk of its
+// keys, a dQ block every key stage of its queries; while the grid is short of
+// the chip, the time is that of the longest block's chain, and fewer rows per
+// wave (16 keys, 32 queries) make its steps shorter and the blocks more.
+// Results are the same bits in causal mode (dK/dV rows are summed over
+// the queries in the same order, dQ rows over the keys).
+// dK/dV with 16 keys per wave pair instead of 32, nb: blocks of 128 keys. It reads
+// Q16 / dO from LDS for half of the MFMAs, 10% slower at D = 64 and 15% at
+// D = 128 once the chip is full. Measured, backward, 32 / 16 keys (dQ at 32
+// queries in both): D = 64: B=4, H=12, T=777 (nb = 336) 60 / 53 us; 1 x 12 x 2048
+// (192) 207 / 172; 4 x 12 x 1024 (384) 70.7 / 71.4; 8 x 12 x 512 (384) 48.5 /
+// 50.3; 1 x 16 x 4096 (512) 223 / 225; 16 x 12 x 1024 (1536) 174 / 192. D = 128:
+// 1 x 16 x 1024 (128) 83 / 70; 1 x 16 x 2048 (256) 143 / 130; 4 x 16 x 512 (256)
+// 59 / 60; 3 x 16 x 1024 (384) 95 / 105. D = 32: 2 x 16 x 2048 (512) 109 / 105;
+// 4 x 16 x 2048 (1024) 168 / 173. Non-causal blocks all have the longest chain
+// and 16 keys gain nothing (4 x 12 x 777, D = 64 74 / 78).
+inline bool bwd_small_dkv(int D, int64_t nb) {
+  const int64_t cus = num_cus();
+  return D == 128 ? nb <= cus : D == 64 ? 2 * nb < 3 * cus : nb <= 2 * cus;
+}
+// dQ with 32 queries per wave (256 per block) instead of 64 (D <= 128), nb: blocks
+// of 512 queries. Measured, backward, 64 / 32 queries per wave: D = 128: 1 x 16 x
+// 2048 (nb = 64) 161 / 143 us; 2 x 16 x 4096 (256) 529 / 502; 1 x 16 x 8192
+// (256) 978 / 935; 8 x 16 x 1024 (256) 199 / 199; 16 x 16 x 512 (256) 147 / 152;
+// 4 x 16 x 4096 (512) 959 / 988. D = 64: 24 x 12 x 512 (288) 132 / 123; 8 x 12 x
+// 2048 (384) 301 / 298; 16 x 12 x 2048 (768) 578 / 576. D = 32: 2 x 16 x 2048 (128) 126 / 108;
+// 8 x 16 x 2048 (512) 301 / 301. Non-causal blocks are equal, so 256 of 512 queries
+// fill the CUs evenly: 4 x 16 x 2048, D = 128 475 / 489.
+inline bool bwd_small_dq(int D, bool causal, int64_t nb, int64_t T) {
+  const int64_t cus = num_cus();
+  if (D == 128) return nb < cus || (causal && nb == cus && T > 512);
+  return 2 * nb <= 3 * cus;
+}
+
+template <typename T, int D, int DE, int MODE, int KR>
+int launch_dkv(const AttnArgs& a, const BwdWs& w, int bh0, int G, int kb0, int nk, hipStream_t st) {
+  constexpr int BK = kNW * KR;  // keys per dK/dV block
+  static_assert((kQB * 64) % BK == 0, "dK/dV blocks tile a band (bands start at multiples of kQB tiles)");
+  const int64_t nb = (std::min<int64_t>((int64_t)(kb0 + nk) * 64, a.T) - (int64_t)kb0 * 64 + BK - 1) / BK;
+  hipLaunchKernelGGL((attn_bwd_dkv_k<T, D, MODE, KR, DE>), dim3((unsigned)(nb * G)), dim3(512), 0, st, a, w.stats,
+                     w.q16, w.qexp, w.ktile, w.kexp, w.dst, bh0, G, kb0, nk);
+  return check_launch("kat_attn_bwd (dkv, mfma)");
+}
+
+template <typename T, int D, int DE, int MODE, int QW>
+int launch_dq(const AttnArgs& a, const BwdWs& w, int bh0, int G, int kb0, int nk, hipStream_t st) {
+  constexpr int BQ = kDqW * QW;  // queries per dQ block
+  // causal: the query blocks wholly before the band have no tiles in it
+  const int64_t nb = (a.T + BQ - 1) / BQ - ((MODE & kModeCausal) ? (int64_t)kb0 * 64 / BQ : 0);
+  hipLaunchKernelGGL((attn_bwd_dq_k<T, D, MODE, DE, QW>), dim3((unsigned)(nb * G)), dim3(64 * kDqW), 0, st, a, w.kexp,
+                     w.ktile, w.dst, bh0, G, kb0, nk, w.dqacc);
+  return check_launch("kat_attn_bwd (dq, mfma)");
+}
+
 template <typename T, int D, int DE, int MODE>
 int launch_bwd(const AttnArgs& a, void* ws, hipStream_t st) {
   constexpr bool kCausal = (MODE & kModeCausal) != 0;
@@ -1540,23 +1574,20 @@ int launch_bwd(const AttnArgs& a, void* ws, hipStream_t st) {
   if (int rc = check_launch("kat_attn_bwd (stats scale)")) return rc;
   // per group of heads (and per band of key tiles): dK, dV (and the dS^T
   // tiles), then dQ from those tiles
-  constexpr int KR = dkv_keys<D>(), BK = kNW * KR;  // keys per wave pair and per dK/dV block
-  static_assert((kQB * 64) % BK == 0, "dK/dV blocks tile a band (bands start at multiples of kQB tiles)");
-  constexpr int BQ = dq_block_queries<D>();                 // queries per dQ block
-  const int nt = (a.T + 63) / 64, nqb = (a.T + BQ - 1) / BQ;
+  const int nt = (a.T + 63) / 64;
   for (int bh0 = 0; bh0 < BH; bh0 += w.group) {
     const int G = std::min(w.group, BH - bh0);
     for (int kb0 = 0; kb0 < nt; kb0 += w.band) {
       const int nk = std::min(w.band, nt - kb0);
-      const int64_t nb = (std::min<int64_t>((int64_t)(kb0 + nk) * 64, a.T) - (int64_t)kb0 * 64 + BK - 1) / BK;
-      // causal: the query blocks wholly before the band have no tiles in it
-      const int64_t nbq = nqb - (kCausal ? (int64_t)kb0 * 64 / BQ : 0);
-      hipLaunchKernelGGL((attn_bwd_dkv_k<T, D, MODE, KR, DE>), dim3((unsigned)(nb * G)), dim3(512), 0, st, a, w.stats,
-                         w.q16, w.qexp, w.ktile, w.kexp, w.dst, bh0, G, kb0, nk);
-      if (int rc = check_launch("kat_attn_bwd (dkv, mfma)")) return rc;
-      hipLaunchKernelGGL((attn_bwd_dq_k<T, D, MODE, DE>), dim3((unsigned)(nbq * G)), dim3(64 * kDqW), 0, st, a,
-                         w.kexp, w.ktile, w.dst, bh0, G, kb0, nk, w.dqacc);
-      if (int rc = check_launch("kat_attn_bwd (dq, mfma)")) return rc;
+      constexpr int KR = dkv_keys<D>(), KRS = kCausal ? 16 : KR;
+      const bool small = KRS < KR && bwd_small_dkv(D, (int64_t)((a.T + 127) / 128) * G);
+      if (int rc = small ? launch_dkv<T, D, DE, MODE, KRS>(a, w, bh0, G, kb0, nk, st)
+                         : launch_dkv<T, D, DE, MODE, KR>(a, w, bh0, G, kb0, nk, st))
+        return rc;
+      if (int rc = bwd_small_dq(D, kCausal, (int64_t)((a.T + 511) / 512) * G, a.T)
+                       ? launch_dq<T, D, DE, MODE, 32>(a, w, bh0, G, kb0, nk, st)
+                       : launch_dq<T, D, DE, MODE, dq_qw<D>()>(a, w, bh0, G, kb0, nk, st))
+        return rc;
     }
   }
   return 0;
