@@ -9,8 +9,8 @@
 // (forward.py:103,126,146) -- on the fp32 matrix instruction instead of the
 // VALU (the tiled kernels in attn_generic.hip: ~3 TFLOP/s at config 1).
 //
-// Block: 4 waves of 16 queries (64 queries; small problems such as config 1,
-// B=2, H=12, S=512, still give 192 blocks). K and V stream through LDS in
+// Block: 4 waves of 16 queries (64 queries; 32 or 16 in grids that do not fill the
+// chip, whose waves split the tiles as well). K and V stream through LDS in
 // tiles of KT keys (64; 32 at D = 128, 16 at D = 256), double-buffered
 // LDS-DMA. Per 16-key
 // group of a tile a wave computes
@@ -69,10 +69,33 @@ template <int M, int NR, int NM> __device__ __forceinline__ void f32_interleave(
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// KG > 1 (small grids, f32_fwd_groups / f32_bwd_groups): a block takes 1 / KG of the rows and its waves
+// form KG groups, wave w in group w / (kF32W / KG), each working every KG-th
+// 16-row group of a tile; the groups' sums are added once at the end, through
+// the (idle) tile buffers. acc: this wave's M pieces; xo: LDS for kF32W M KB;
+// os: the totals of pieces kg M / KG .. of the wave's rows (in group order:
+// deterministic). The caller synchronises before xo is used again.
+template <int KG, int M>
+__device__ __forceinline__ void f32_add_groups(const f32x4 (&acc)[M], f32x4* xo, int w, int lane, f32x4 (&os)[M / KG]) {
+  constexpr int RG = kF32W / KG;  // waves (row sets) per group
+#pragma unroll
+  for (int m = 0; m < M; ++m) xo[(w * M + m) * 64 + lane] = acc[m];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < M / KG; ++i) {
+    const int m = (w / RG) * (M / KG) + i;
+    f32x4 t = xo[((w % RG) * M + m) * 64 + lane];
+#pragma unroll
+    for (int k = 1; k < KG; ++k) t += xo[((k * RG + w % RG) * M + m) * 64 + lane];
+    os[i] = t;
+  }
+}
+
 // D = 256: one block per CU (one wave per SIMD, 512 registers: the Q fragments
 // and O accumulators take 128)
-template <int D, int MODE>
+template <int D, int MODE, int KG>
 __global__ __launch_bounds__(64 * kF32W, D >= 256 ? 1 : 2) void attn_fwd_f32_k(AttnArgs a) {
+  constexpr int BM = kF32BM / KG;  // queries per block
   constexpr int D16 = 2 * D;  // a row in 16-bit units, the unit of the tile helpers
   constexpr int KT = f32_kt<D>();
   constexpr int M = D / 16;  // 16-column blocks of d: 4 k-steps of QK^T each; O^T subtiles
@@ -85,12 +108,13 @@ __global__ __launch_bounds__(64 * kF32W, D >= 256 ? 1 : 2) void attn_fwd_f32_k(A
   const int T_ = a.T, H = a.H;
   int bh, rank;
   block_order((int)blockIdx.x, a.B * H, bh, rank);
-  const int n_qt = (T_ + kF32BM - 1) / kF32BM;
-  const int q0 = (n_qt - 1 - rank) * kF32BM;
+  const int n_qt = (T_ + BM - 1) / BM;
+  const int q0 = (n_qt - 1 - rank) * BM;
   const int b = bh / H, h = bh - b * H;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 4, li = lane & 15;
-  const int qw = q0 + kF32Q * w;
+  const int kg = KG == 1 ? 0 : w / (kF32W / KG);
+  const int qw = q0 + kF32Q * (KG == 1 ? w : w % (kF32W / KG));
 
   const float* qp = (const float*)a.q + b * a.sq[0] + h * a.sq[1];
   const float* kp = (const float*)a.k + b * a.sk[0] + h * a.sk[1];
@@ -171,7 +195,8 @@ __global__ __launch_bounds__(64 * kF32W, D >= 256 ? 1 : 2) void attn_fwd_f32_k(A
   };
   auto tile = [&](auto masked_tag, int k0, const short* ks_, const short* vs_) __attribute__((always_inline)) {
 #pragma unroll
-    for (int hr = 0; hr < KT; hr += 16) group(masked_tag, hr, k0 + hr, ks_, vs_);
+    for (int hr = 0; hr < KT; hr += 16 * KG)
+      group(masked_tag, hr, k0 + 16 * kg + hr, ks_ + 16 * kg * D16, vs_ + 16 * kg * D16);
   };
   // which variant a tile takes (as in the bf16 forward): causal without a
   // padding mask -- below the diagonal plain, straddling it masked, above it
@@ -195,7 +220,7 @@ __global__ __launch_bounds__(64 * kF32W, D >= 256 ? 1 : 2) void attn_fwd_f32_k(A
     }
   };
 
-  const int n_kt = kCausal ? (std::min(q0 + kF32BM, T_) + KT - 1) / KT : (T_ + KT - 1) / KT;
+  const int n_kt = kCausal ? (std::min(q0 + BM, T_) + KT - 1) / KT : (T_ + KT - 1) / KT;
   // this lane's padding-mask byte of key tile kt (0 past the tile or the end)
   auto kmbyte = [&](int kt) __attribute__((always_inline)) {
     const int j = kt * KT + lane;
@@ -233,16 +258,29 @@ __global__ __launch_bounds__(64 * kF32W, D >= 256 ? 1 : 2) void attn_fwd_f32_k(A
   float l = lsum;
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
+  f32x4 os[M / KG];
+  if constexpr (KG == 1) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) os[m] = oacc[m];
+  } else {
+    static_assert(M % KG == 0 && KT % (16 * KG) == 0 && sizeof(sk) >= kF32W * M * 1024, "split");
+    float* const xl = reinterpret_cast<float*>(&sv[0][0]);
+    if (g == 0) xl[w * 16 + li] = l;
+    f32_add_groups<KG>(oacc, reinterpret_cast<f32x4*>(&sk[0][0]), w, lane, os);
+    l = xl[(w % (kF32W / KG)) * 16 + li];
+#pragma unroll
+    for (int q = 1; q < KG; ++q) l += xl[(q * (kF32W / KG) + w % (kF32W / KG)) * 16 + li];
+  }
   const int qrow = qw + li;
   if (qrow >= T_) return;
   const float inv = 1.f / (l + 16.f * a.eps);
   float* __restrict__ Lp = a.L + b * a.sl[0] + h * a.sl[1];
-  if (g == 0) Lp[(int64_t)qrow * a.sl[2]] = l * 0.0625f;
+  if (g == 0 && kg == 0) Lp[(int64_t)qrow * a.sl[2]] = l * 0.0625f;
   float* __restrict__ op = (float*)a.o + b * a.so[0] + h * a.so[1] + (int64_t)qrow * a.so[2];
 #pragma unroll
-  for (int m = 0; m < M; ++m) {
-    const int col = 16 * m + 4 * g;
-    if (col < DR) *reinterpret_cast<f32x4*>(op + col) = oacc[m] * inv;
+  for (int m = 0; m < M / KG; ++m) {
+    const int col = 16 * (kg * (M / KG) + m) + 4 * g;
+    if (col < DR) *reinterpret_cast<f32x4*>(op + col) = os[m] * inv;
   }
 }
 
@@ -292,9 +330,10 @@ template <int D> union F32BwdSmem {
 };
 
 // bid: the block's index among the dQ blocks
-template <int D, int MODE>
+template <int D, int MODE, int KG>
 __device__ __forceinline__ void bwd_dq_f32(const AttnArgs& a, const float* __restrict__ delta,
                                            const float* __restrict__ cinv, int bid, F32DqSmem<D>& sm) {
+  constexpr int BM = kF32BM / KG;  // queries per block
   constexpr int D16 = 2 * D;
   constexpr int KT = f32_kt<D>();
   constexpr int M = D / 16;
@@ -307,12 +346,13 @@ __device__ __forceinline__ void bwd_dq_f32(const AttnArgs& a, const float* __res
   const int T_ = a.T, H = a.H;
   int bh, rank;
   block_order(bid, a.B * H, bh, rank);
-  const int n_qt = (T_ + kF32BM - 1) / kF32BM;
-  const int q0 = (n_qt - 1 - rank) * kF32BM;
+  const int n_qt = (T_ + BM - 1) / BM;
+  const int q0 = (n_qt - 1 - rank) * BM;
   const int b = bh / H, h = bh - b * H;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 4, li = lane & 15;
-  const int qw = q0 + kF32Q * w;
+  const int kg = KG == 1 ? 0 : w / (kF32W / KG);
+  const int qw = q0 + kF32Q * (KG == 1 ? w : w % (kF32W / KG));
 
   const float* qp = (const float*)a.q + b * a.sq[0] + h * a.sq[1];
   const float* kp = (const float*)a.k + b * a.sk[0] + h * a.sk[1];
@@ -396,7 +436,8 @@ __device__ __forceinline__ void bwd_dq_f32(const AttnArgs& a, const float* __res
   };
   auto tile = [&](auto masked_tag, int k0, const short* ks_, const short* vs_) __attribute__((always_inline)) {
 #pragma unroll
-    for (int hr = 0; hr < KT; hr += 16) group(masked_tag, hr, k0 + hr, ks_, vs_);
+    for (int hr = 0; hr < KT; hr += 16 * KG)
+      group(masked_tag, hr, k0 + 16 * kg + hr, ks_ + 16 * kg * D16, vs_ + 16 * kg * D16);
   };
   auto tile_step = [&](int k0, const short* ks_, const short* vs_) __attribute__((always_inline)) {
     if constexpr (kCausal && !kKM) {
@@ -416,7 +457,7 @@ __device__ __forceinline__ void bwd_dq_f32(const AttnArgs& a, const float* __res
     }
   };
 
-  const int n_kt = kCausal ? (std::min(q0 + kF32BM, T_) + KT - 1) / KT : (T_ + KT - 1) / KT;
+  const int n_kt = kCausal ? (std::min(q0 + BM, T_) + KT - 1) / KT : (T_ + KT - 1) / KT;
   auto kmbyte = [&](int kt) __attribute__((always_inline)) {
     const int j = kt * KT + lane;
     return (kKM && lane < KT && j < T_) ? (uint32_t)kmb[j] : 0u;
@@ -448,21 +489,30 @@ __device__ __forceinline__ void bwd_dq_f32(const AttnArgs& a, const float* __res
     step(kt, std::integral_constant<int, 0>{});
     if (kt + 1 < n_kt) step(kt + 1, std::integral_constant<int, 1>{});
   }
+  f32x4 os[M / KG];
+  if constexpr (KG == 1) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) os[m] = qacc[m];
+  } else {
+    static_assert(M % KG == 0 && KT % (16 * KG) == 0 && sizeof(sk) >= kF32W * M * 1024, "split");
+    f32_add_groups<KG>(qacc, reinterpret_cast<f32x4*>(&sk[0][0]), w, lane, os);
+  }
   if (!qin) return;
   float* __restrict__ dqp = (float*)a.dq + b * a.sdq[0] + h * a.sdq[1] + (int64_t)qrow * a.sdq[2];
 #pragma unroll
-  for (int m = 0; m < M; ++m) {
-    const int col = 16 * m + 4 * g;
-    if (col < DR) *reinterpret_cast<f32x4*>(dqp + col) = qacc[m] * scale;
+  for (int m = 0; m < M / KG; ++m) {
+    const int col = 16 * (kg * (M / KG) + m) + 4 * g;
+    if (col < DR) *reinterpret_cast<f32x4*>(dqp + col) = os[m] * scale;
   }
 }
 
 // D = 256: the K^T and V^T fragments and the dV^T and dK^T accumulators alone
 // take 256 VGPRs, so one block per CU (one wave per SIMD, 512 registers)
 // bid: the block's index among the dK/dV blocks
-template <int D, int MODE>
+template <int D, int MODE, int KG>
 __device__ __forceinline__ void bwd_dkv_f32(const AttnArgs& a, const float* __restrict__ delta,
                                             const float* __restrict__ cinv, int bid, F32DkvSmem<D>& sm) {
+  constexpr int KB = kF32KB / KG;  // keys per block
   constexpr int D16 = 2 * D;
   constexpr int QT = f32_qt<D>();
   constexpr int M = D / 16;
@@ -475,11 +525,12 @@ __device__ __forceinline__ void bwd_dkv_f32(const AttnArgs& a, const float* __re
   const int T_ = a.T, H = a.H;
   int bh, rank;
   block_order(bid, a.B * H, bh, rank);  // rank 0: the first keys (most queries)
-  const int k0 = rank * kF32KB;
+  const int k0 = rank * KB;
   const int b = bh / H, h = bh - b * H;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 4, li = lane & 15;
-  const int kw = k0 + 16 * w;  // this wave's 16 keys
+  const int kg = KG == 1 ? 0 : w / (kF32W / KG);  // the wave's group (of query rows)
+  const int kw = k0 + 16 * (KG == 1 ? w : w % (kF32W / KG));  // this wave's 16 keys
   const int key = kw + li;     // lane (g, li): key li of the wave, queries 4 g + jj of a group
 
   const float* qp = (const float*)a.q + b * a.sq[0] + h * a.sq[1];
@@ -571,9 +622,9 @@ __device__ __forceinline__ void bwd_dkv_f32(const AttnArgs& a, const float* __re
   // after one of the wave's keys)
   auto tile = [&](int q0t, const short* qs_, const short* gs_, const float* st_) __attribute__((always_inline)) {
 #pragma unroll
-    for (int hr = 0; hr < QT; hr += 16) {
-      const int qh = q0t + hr;
-      if (!kCausal || qh + 15 >= kw) group(hr, qh, qs_, gs_, st_);
+    for (int hr = 0; hr < QT; hr += 16 * KG) {
+      const int qh = q0t + 16 * kg + hr;
+      if (!kCausal || qh + 15 >= kw) group(hr, qh, qs_ + 16 * kg * D16, gs_ + 16 * kg * D16, st_ + 16 * kg);
     }
   };
 
@@ -612,16 +663,28 @@ __device__ __forceinline__ void bwd_dkv_f32(const AttnArgs& a, const float* __re
     if (qt + 1 < n_qt) step(qt + 1, std::integral_constant<int, 1>{});
   }
 
+  f32x4 ov[M / KG], ok[M / KG];
+  if constexpr (KG == 1) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      ov[m] = vacc[m];
+      ok[m] = kacc[m];
+    }
+  } else {
+    static_assert(M % KG == 0 && QT % (16 * KG) == 0 && sizeof(sq) >= kF32W * M * 1024, "split");
+    f32_add_groups<KG>(vacc, reinterpret_cast<f32x4*>(&sq[0][0]), w, lane, ov);
+    f32_add_groups<KG>(kacc, reinterpret_cast<f32x4*>(&sg[0][0]), w, lane, ok);
+  }
   if (key >= T_) return;
   const bool kin = !kKM || a.km[(int64_t)b * a.skm + key] != 0;  // a dropped key's gradients are 0
   float* __restrict__ dvp = (float*)a.dv + b * a.sdv[0] + h * a.sdv[1] + (int64_t)key * a.sdv[2];
   float* __restrict__ dkp = (float*)a.dk + b * a.sdk[0] + h * a.sdk[1] + (int64_t)key * a.sdk[2];
 #pragma unroll
-  for (int m = 0; m < M; ++m) {
-    const int col = 16 * m + 4 * g;
+  for (int m = 0; m < M / KG; ++m) {
+    const int col = 16 * (kg * (M / KG) + m) + 4 * g;
     if (col < DR) {
-      *reinterpret_cast<f32x4*>(dvp + col) = kin ? vacc[m] : f32x4{0.f, 0.f, 0.f, 0.f};
-      *reinterpret_cast<f32x4*>(dkp + col) = kin ? kacc[m] * scale : f32x4{0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<f32x4*>(dvp + col) = kin ? ov[m] : f32x4{0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<f32x4*>(dkp + col) = kin ? ok[m] * scale : f32x4{0.f, 0.f, 0.f, 0.f};
     }
   }
 }
@@ -633,15 +696,15 @@ __device__ __forceinline__ void bwd_dkv_f32(const AttnArgs& a, const float* __re
 // for block_order. Small problems run both parts side by side (config 1,
 // B=2, H=12, S=512: 192 + 192 blocks on 256 CUs) instead of one after the
 // other; the LDS of the two parts is shared, registers are the larger part's.
-template <int D, int MODE>
+template <int D, int MODE, int KG>
 __global__ __launch_bounds__(64 * kF32W, D >= 256 ? 1 : 2) void attn_bwd_f32_k(AttnArgs a, const float* __restrict__ delta,
                                                               const float* __restrict__ cinv, int nk, int nkp) {
   __shared__ F32BwdSmem<D> sm;
   const int id = (int)blockIdx.x;
   if (id < nk)
-    bwd_dkv_f32<D, MODE>(a, delta, cinv, id, sm.dkv);
+    bwd_dkv_f32<D, MODE, KG>(a, delta, cinv, id, sm.dkv);
   else if (id >= nkp)
-    bwd_dq_f32<D, MODE>(a, delta, cinv, id - nkp, sm.dq);
+    bwd_dq_f32<D, MODE, KG>(a, delta, cinv, id - nkp, sm.dq);
 }
 
 // layout widths of the fp32 kernels: 32, 64, 128, 256 (a head dim between
@@ -656,20 +719,70 @@ int f32_width(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256
     default: { constexpr int MODE = 0; __VA_ARGS__; }                                   \
   }
 
-template <int D, int MODE> int launch_fwd_f32(const AttnArgs& a, hipStream_t st) {
-  const int64_t nb = (int64_t)((a.T + kF32BM - 1) / kF32BM) * a.B * a.H;
-  hipLaunchKernelGGL((attn_fwd_f32_k<D, MODE>), dim3((unsigned)nb), dim3(64 * kF32W), 0, st, a);
-  return check_launch("kat_attn_fwd (fp32 mfma)");
+// Wave groups per block (KG) for a grid of nb blocks of 64 rows. While the grid is
+// short of the chip, the time is the longest block's chain of MFMAs and LDS
+// waits; splitting a block's tiles over its waves halves or quarters it and
+// makes as many more blocks. It costs tile loads per row and the final sums,
+// so full grids keep one group. Measured, 1 / 2 / 4 groups, us: forward, D = 64:
+// B=2, H=12, T=512 (nb = 192) 24.6 / 18.1 / 16.5; 1 x 12 x 1024 (192) 45.7 / 32.1 /
+// 25.1; 1 x 20 x 1024 (320) 51.3 / 34.4 / 36.9; 2 x 12 x 1024 (384) 54.9 / 40.9 /
+// 41.2; 4 x 12 x 1024 (768) 71.9 / 68.8 / 78.5; 4 x 16 x 2048 (2048) 306 / 324 /
+// 365; 8 x 16 x 128 (256) 9.1 / 8.1 / 10.4; 16 x 12 x 128 (384) 11.6 / 13.0 / 14.7;
+// D = 128: 2 x 12 x 512 (192) 41.7 / 30.7; D = 32: 16.4 / 11.5; non-causal D = 64:
+// 2 x 16 x 512 (256) 25.0 / 24.0 / 27.2; 1 x 12 x 1024 (192) 45.7 / 43.1 / 38.7.
+int f32_fwd_groups(int D, bool causal, int64_t nb, int64_t T) {
+  const int64_t cus = num_cus();
+  if (D > 128) return 1;
+  if (D == 64 && (2 * nb <= cus || (T > 256 && (causal ? nb <= cus : 4 * nb <= 3 * cus)))) return 4;
+  return nb <= cus || (T > 128 && nb <= 3 * cus) ? 2 : 1;
+}
+// The same for the backward's two kinds of blocks (nb of each). D = 64: 2 x 12 x 512
+// (192) 62.5 / 40.4 / 43.6; 1 x 10 x 1024 (160) 104 / 66 / 60; 1 x 8 x 1024 (128)
+// 86.4 / 70.2 / 47.4; 1 x 20 x 1024 (320) 121 / 105 / 108; 8 x 12 x 256 (384) 43.8 /
+// 46.1 / 53.9; 2 x 12 x 1024 (384) 120 / 121 / 128; D = 128: 1 x 12 x 1024 (192)
+// 213 / 117; D = 32: 2 x 12 x 512 (192) 38 / 27; non-causal: D = 64, 1 x 12 x 1024
+// (192) 130 / 111 / 112, D = 128, 1 x 16 x 1024 (256) 245 / 250.
+int f32_bwd_groups(int D, bool causal, int64_t nb) {
+  const int64_t cus = num_cus();
+  if (D > 128) return 1;
+  if (!causal) return 4 * nb <= 3 * cus ? 2 : 1;
+  if (D == 64 && 8 * nb <= 5 * cus) return 4;
+  return nb <= cus ? 2 : 1;
 }
 
-template <int D, int MODE>
-int launch_bwd_f32(const AttnArgs& a, const float* delta, const float* cinv, hipStream_t st) {
-  const int64_t nq = (int64_t)((a.T + kF32BM - 1) / kF32BM) * a.B * a.H;
-  const int64_t nk = (int64_t)((a.T + kF32KB - 1) / kF32KB) * a.B * a.H;
+template <int D, int MODE, int KG> int launch_fwd_f32_kg(const AttnArgs& a, hipStream_t st) {
+  constexpr int BM = kF32BM / KG;
+  const int64_t nb = (int64_t)((a.T + BM - 1) / BM) * a.B * a.H;
+  hipLaunchKernelGGL((attn_fwd_f32_k<D, MODE, KG>), dim3((unsigned)nb), dim3(64 * kF32W), 0, st, a);
+  return check_launch("kat_attn_fwd (fp32 mfma)");
+}
+template <int D, int MODE> int launch_fwd_f32(const AttnArgs& a, hipStream_t st) {
+  const int kg = f32_fwd_groups(D, (MODE & kModeCausalF) != 0, (int64_t)((a.T + kF32BM - 1) / kF32BM) * a.B * a.H, a.T);
+  if constexpr (D == 64)
+    if (kg == 4) return launch_fwd_f32_kg<D, MODE, 4>(a, st);
+  if constexpr (D <= 128)
+    if (kg == 2) return launch_fwd_f32_kg<D, MODE, 2>(a, st);
+  return launch_fwd_f32_kg<D, MODE, 1>(a, st);
+}
+
+template <int D, int MODE, int KG>
+int launch_bwd_f32_kg(const AttnArgs& a, const float* delta, const float* cinv, hipStream_t st) {
+  constexpr int BM = kF32BM / KG, KB = kF32KB / KG;
+  const int64_t nq = (int64_t)((a.T + BM - 1) / BM) * a.B * a.H;
+  const int64_t nk = (int64_t)((a.T + KB - 1) / KB) * a.B * a.H;
   const int64_t nkp = (nk + 7) & ~(int64_t)7;
-  hipLaunchKernelGGL((attn_bwd_f32_k<D, MODE>), dim3((unsigned)(nkp + nq)), dim3(64 * kF32W), 0, st, a, delta,
+  hipLaunchKernelGGL((attn_bwd_f32_k<D, MODE, KG>), dim3((unsigned)(nkp + nq)), dim3(64 * kF32W), 0, st, a, delta,
                      cinv, (int)nk, (int)nkp);
   return check_launch("kat_attn_bwd (fp32 mfma)");
+}
+template <int D, int MODE>
+int launch_bwd_f32(const AttnArgs& a, const float* delta, const float* cinv, hipStream_t st) {
+  const int kg = f32_bwd_groups(D, (MODE & kModeCausalF) != 0, (int64_t)((a.T + kF32BM - 1) / kF32BM) * a.B * a.H);
+  if constexpr (D == 64 && (MODE & kModeCausalF) != 0)
+    if (kg == 4) return launch_bwd_f32_kg<D, MODE, 4>(a, delta, cinv, st);
+  if constexpr (D <= 128)
+    if (kg == 2) return launch_bwd_f32_kg<D, MODE, 2>(a, delta, cinv, st);
+  return launch_bwd_f32_kg<D, MODE, 1>(a, delta, cinv, st);
 }
 
 // 31-bit byte offsets per (b, h) slice for every row the kernels address
