@@ -325,7 +325,14 @@ template <typename A> __device__ __forceinline__ A pair_sum(const A (&a)[4]) { r
 // FULL: the row is exactly NCH chunk rounds long, so every chunk is in range
 // and the column tests fold away (the norm kernels take this when it holds).
 // TPR: threads per row, 256 (the block's) or 64 (one wave's).
-template <int TPR> __device__ __forceinline__ int row_tid() { return (int)threadIdx.x & (TPR - 1); }
+template <int TPR> __device__ __forceinline__ int row_tid() { return TPR == 256 ? (int)threadIdx.x : (int)threadIdx.x & (TPR - 1); }
+// The row a thread starts at: a scalar, as every thread of a block (or wave) has
+// the same. Left to the compiler as threadIdx.x / TPR, the rows and their
+// addresses take vector registers: 10-18 more, or spills.
+template <int TPR> __device__ __forceinline__ int64_t first_row() {
+  if constexpr (TPR == 256) return blockIdx.x;
+  return (int64_t)blockIdx.x * (256 / TPR) + __builtin_amdgcn_readfirstlane((int)threadIdx.x / TPR);
+}
 template <typename T, int NCH, bool FULL = false, int TPR = 256>
 __device__ __forceinline__ void load_row(const T* __restrict__ base, int n_cols, VecT<T, Raw<T>::V> (&r)[NCH]) {
   constexpr int V = Raw<T>::V;
@@ -706,7 +713,7 @@ __global__ __launch_bounds__(256) void men_fwd_k(const T* __restrict__ x, const 
   load_weight<T, W, NCH, TPR>(w, n_cols, wv);
   constexpr int RPB = 256 / TPR;  // rows per block at a time
   const int64_t G = (int64_t)gridDim.x * RPB;
-  int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / TPR;
+  int64_t row = first_row<TPR>();
   const int64_t last = n_rows - 1;
   VecT<T, V> cur[NCH], nx1[NCH];
   VecT<RT, V> rc[NCH], r1[NCH];
@@ -797,7 +804,7 @@ __global__ __launch_bounds__(256) void men_bwd_k(
   const A e = A(eps);
   constexpr int RPB = 256 / TPR;  // rows per block at a time
   const int64_t G = (int64_t)gridDim.x * RPB;
-  int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / TPR;
+  int64_t row = first_row<TPR>();
   // ring of rows row, row + G, ..., row + PF*G: slot 0 is reduced next
   VecT<Y, V> by[PF + 1][NCH];
   VecT<T, V> bx[PF + 1][NCH], bh[PF + 1][NCH];
