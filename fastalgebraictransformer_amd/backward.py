@@ -33,6 +33,10 @@ def _attn_bwd_into(q, k, v, output, L, grad_output, dq, dk, dv, alibi_slopes, sc
     allocator. ``extended``: kat_attn_bwd_masked (see _attn_fwd_into)."""
     lib = _lib.load()
     B, H, T, D = q.shape
+    if key_mask is not None:  # saved by the forward as uint8 [B, T]; a hook may return it otherwise
+        if key_mask.device != q.device or key_mask.dtype != torch.uint8 or key_mask.shape != (B, T):
+            raise RuntimeError("backward: the saved key mask must be uint8 [B, T] on the inputs' device")
+        key_mask = key_mask.contiguous()
     _warn_if_tiled((q, k, v, output, grad_output, dq, dk, dv), D, q.dtype,
                    mfma_inputs=(q, k, v, output, grad_output))
     slopes = alibi_slopes.to(device=q.device, dtype=torch.float32).contiguous()

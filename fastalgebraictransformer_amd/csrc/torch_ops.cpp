@@ -417,6 +417,16 @@ void python_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor&
                               km.defined() ? py::cast(km) : none, extended);
 }
 
+// the key mask a backward unpacked (undefined: none) as the kernels read it:
+// uint8, rows of T bytes
+Tensor saved_mask(const Tensor& q, const Tensor& km, int64_t B, int64_t T) {
+  if (!km.defined()) return km;
+  if (!km.is_cuda() || km.device() != q.device() || km.layout() != at::kStrided || km.scalar_type() != at::kByte ||
+      km.sizes() != at::IntArrayRef({B, T}))
+    throw std::runtime_error("backward: the saved key mask must be uint8 [B, T] on the inputs' CUDA device");
+  return km.contiguous();
+}
+
 // a [B, T] key mask as uint8 (nonzero = attend), a copy of the caller's
 struct Mask {
   Tensor t;  // undefined: no mask
@@ -453,7 +463,7 @@ struct Attention : Function<Attention> {
     need(s[0], {&s[1], &s[2], &s[3], &s[4], &s[5], &gr[0]});
     const at::ScalarType dt = s[0].scalar_type();
     const Tensor &q = s[0], k = as(s[1], dt), v = as(s[2], dt), o = as(s[3], dt), L = as(s[4], at::kFloat);
-    const Tensor &slopes = s[5], &km = s[6];
+    const Tensor &slopes = s[5], km = saved_mask(q, s[6], q.size(0), q.size(2));
     const double scale = ctx->saved_data["scale"].toDouble(), eps = ctx->saved_data["eps"].toDouble();
     const bool extended = ctx->saved_data["extended"].toBool(), causal = ctx->saved_data["causal"].toBool();
     const Dims n{q.size(0), q.size(1), q.size(2), q.size(3)};
@@ -509,7 +519,8 @@ struct PackedAttention : Function<PackedAttention> {
   static variable_list backward(AutogradContext* ctx, variable_list gr) {
     const auto s = ctx->get_saved_variables();
     need(s[0], {&s[1], &s[2], &s[3], &gr[0]});
-    const Tensor &qkv = s[0], y = as(s[1], qkv.scalar_type()), L = as(s[2], at::kFloat), &slopes = s[3], &km = s[4];
+    const Tensor &qkv = s[0], y = as(s[1], qkv.scalar_type()), L = as(s[2], at::kFloat), &slopes = s[3];
+    const Tensor km = saved_mask(qkv, s[4], qkv.size(0), qkv.size(1));
     const double scale = ctx->saved_data["scale"].toDouble(), eps = ctx->saved_data["eps"].toDouble();
     const Dims n{qkv.size(0), qkv.size(3), qkv.size(1), qkv.size(4)};
     Tensor go = as(gr[0], qkv.scalar_type());

@@ -207,6 +207,43 @@ def test_saved_tensor_hooks_and_checkpoint(gpu):
             torch.autograd.grad(y, leaves, torch.ones_like(y))
 
 
+def _masked_ops(D):
+    q = [_rand(i, 3, 2, 70, D, dtype=torch.bfloat16) for i in range(3)]
+    slopes = F.compute_alibi_slopes(2).cuda()
+    km = torch.rand(3, 70, generator=torch.Generator().manual_seed(2)).cuda() > 0.4
+    cls, pcls = F.backward.MaskedRationalAttentionFunction, F.backward.PackedRationalAttention
+    return [("masked", lambda a, b, c: F.rational_attention_masked(a, b, c, slopes, 0.125, km), q),
+            ("masked class", lambda a, b, c: cls.apply(a, b, c, slopes, 0.125, km, True, 1e-6), q),
+            ("packed", lambda a: F.rational_attention_packed(a, slopes, 0.125, key_mask=km),
+             [_rand(5, 3, 70, 3, 2, D, dtype=torch.bfloat16)]),
+            ("packed class", lambda a: pcls.apply(a, slopes, 0.125, 1e-6, km),
+             [_rand(5, 3, 70, 3, 2, D, dtype=torch.bfloat16)])]
+
+
+@pytest.mark.filterwarnings("ignore:rational attention in")
+@pytest.mark.parametrize("D", [64, 20])  # the MFMA kernels, and a head dim outside them
+def test_saved_key_mask_of_another_layout_or_place(gpu, D):
+    """Only the mask comes back changed from a saved-tensor hook: with a row
+    stride it gives the same gradients; on the host, in another dtype or with
+    other sizes it raises before any launch."""
+    def mask_only(change):
+        return torch.autograd.graph.saved_tensors_hooks(
+            lambda t: t, lambda t: change(t) if t.dtype == torch.uint8 else t)
+
+    def strided(t):
+        return torch.zeros(t.shape[0], t.shape[1] + 9, dtype=t.dtype, device="cuda")[:, :t.shape[1]].copy_(t)
+
+    for name, fn, ins in _masked_ops(D):
+        _, g0 = _plain_grads(fn, ins)
+        for change in (strided, lambda t: t.t().contiguous().t()):
+            with mask_only(change):
+                _, g = _plain_grads(fn, ins)
+            assert all(torch.equal(a, b) for a, b in zip(g, g0)), name
+        for change in (lambda t: t.cpu(), lambda t: t.float(), lambda t: t[:, :-1], lambda t: t[:1]):
+            with mask_only(change), pytest.raises(RuntimeError, match="saved key mask"):
+                _plain_grads(fn, ins)
+
+
 def test_modes_and_partial_gradients(gpu):
     for name, fn, ins in _ops_list():
         y0, g0 = _plain_grads(fn, ins)
