@@ -122,6 +122,15 @@ def check(rc, name):
         raise RuntimeError(f"{name} failed (status {rc}): {msg}")
 
 
+def need(a, *wanted):
+    """What a backward unpacked or was handed: ``a`` and (tensor, shape) pairs on
+    its CUDA device; raise before a launch that would read past them."""
+    for t, shape in wanted:
+        if not a.is_cuda or t.device != a.device or t.shape != shape:
+            raise RuntimeError("backward: saved tensors and gradients must be tensors of one CUDA "
+                               "device with the sizes of the forward")
+
+
 def i64_array(values):
     arr = (ctypes.c_int64 * len(values))(*[int(x) for x in values])
     return arr

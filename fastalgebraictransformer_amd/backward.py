@@ -29,10 +29,17 @@ from .forward import (  # noqa: F401
 def _attn_bwd_into(q, k, v, output, L, grad_output, dq, dk, dv, alibi_slopes, scale, causal, eps,
                    key_mask=None, extended=False):
     """Launch the attention backward; every [B,H,T,D] argument may have any
-    (b, h, t) strides with a unit d-stride. The workspace comes from torch's
-    allocator. ``extended``: kat_attn_bwd_masked (see _attn_fwd_into)."""
+    (b, h, t) strides (a copy is made of an input whose d-stride is not 1). The
+    workspace comes from torch's allocator. ``extended``: kat_attn_bwd_masked
+    (see _attn_fwd_into)."""
     lib = _lib.load()
     B, H, T, D = q.shape
+    # what saved-tensor hooks return may differ from what the forward saved
+    q = _unit_d(q)
+    k, v, output, grad_output = (_unit_d(t.to(q.dtype)) for t in (k, v, output, grad_output))
+    L = L.to(torch.float32)
+    _lib.need(q, (k, q.shape), (v, q.shape), (output, q.shape), (grad_output, q.shape),
+              (L, (B, H, T) + L.shape[3:]))
     if key_mask is not None:  # saved by the forward as uint8 [B, T]; a hook may return it otherwise
         if key_mask.device != q.device or key_mask.dtype != torch.uint8 or key_mask.shape != (B, T):
             raise RuntimeError("backward: the saved key mask must be uint8 [B, T] on the inputs' device")
@@ -40,6 +47,8 @@ def _attn_bwd_into(q, k, v, output, L, grad_output, dq, dk, dv, alibi_slopes, sc
     _warn_if_tiled((q, k, v, output, grad_output, dq, dk, dv), D, q.dtype,
                    mfma_inputs=(q, k, v, output, grad_output))
     slopes = alibi_slopes.to(device=q.device, dtype=torch.float32).contiguous()
+    if slopes.numel() < H:
+        raise RuntimeError("backward: alibi_slopes must have n_heads entries")
     code = _lib.dtype_code(q)
     if extended:
         ws_bytes = lib.kat_attn_bwd_masked_workspace_size(B, H, T, D, code, int(bool(causal)))
@@ -73,9 +82,6 @@ def rational_attention_backward(q, k, v, output, L, grad_output, alibi_slopes, s
     assert q.is_cuda
     B, H, T, D = q.shape
     dt = q.dtype
-    k, v, output, grad_output = (t.to(dt) for t in (k, v, output, grad_output))
-    q, k, v, output, grad_output = (_unit_d(t) for t in (q, k, v, output, grad_output))
-    L = L.to(torch.float32)
     dq = torch.empty((B, H, T, D), dtype=dt, device=q.device)
     dk = torch.empty((B, H, T, D), dtype=dt, device=q.device)
     dv = torch.empty((B, H, T, D), dtype=dt, device=q.device)

@@ -79,11 +79,19 @@ void check(int rc, const char* name) {
     throw std::runtime_error(std::string(name) + " failed (status " + std::to_string(rc) + "): " + kat_last_error());
 }
 
-// what a backward unpacked or was handed: device tensors, or no launch
-void need(const Tensor& a, std::initializer_list<const Tensor*> ts) {
+// What a backward unpacked (a hook may return another tensor than it was given)
+// or was handed: `a` and tensors on its device of the sizes the launch reads, or
+// no launch. Call it on what as() returned, whose dtypes are the launch's.
+struct Want {
+  const Tensor& t;
+  at::IntArrayRef sizes;
+};
+void need(const Tensor& a, std::initializer_list<Want> ts) {
   bool ok = plain(a);
-  for (const Tensor* t : ts) ok = ok && t->defined() && t->is_cuda() && t->device() == a.device();
-  if (!ok) throw std::runtime_error("backward: saved tensors and gradients must be tensors of one CUDA device");
+  for (const Want& w : ts) ok = ok && plain(w.t) && w.t.device() == a.device() && w.t.sizes() == w.sizes;
+  if (!ok)
+    throw std::runtime_error(
+        "backward: saved tensors and gradients must be tensors of one CUDA device with the sizes of the forward");
 }
 
 void* stream(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
@@ -124,7 +132,10 @@ struct Rows {
   }
 };
 
-Tensor as(const Tensor& t, at::ScalarType dt) { return t.scalar_type() == dt ? t : t.to(dt); }
+Tensor as(const Tensor& t, at::ScalarType dt) {
+  const Tensor r = t.is_neg() ? t.resolve_neg() : t;
+  return r.scalar_type() == dt ? r : r.to(dt);
+}
 
 Tensor bytes(size_t n, const Tensor& like) {
   return at::empty({(int64_t)std::max<size_t>(n, 1)}, like.options().dtype(at::kByte));
@@ -146,9 +157,9 @@ struct Softmax : Function<Softmax> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &x = saved[0], &out = saved[1];
-    need(x, {&out, &g[0]});
-    const Rows rx(x), rp(out), rg(as(g[0], x.scalar_type()));
+    const Tensor &x = saved[0], out = as(saved[1], x.scalar_type()), dy = as(g[0], x.scalar_type());
+    need(x, {{out, x.sizes()}, {dy, x.sizes()}});
+    const Rows rx(x), rp(out), rg(dy);
     Tensor dx = at::empty(x.sizes(), x.options().memory_format(at::MemoryFormat::Contiguous));
     check(kat_rsoftmax_bwd(rg.p(), rx.p(), rp.p(), dx.data_ptr(), rx.rows, rx.cols, rg.ld, rx.ld, rp.ld, rx.cols,
                            (float)ctx->saved_data["eps"].toDouble(), code(x), stream(x)),
@@ -173,9 +184,9 @@ struct Swiglu : Function<Swiglu> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list gr) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor& gate = saved[0];
-    need(gate, {&saved[1], &gr[0]});
-    const Rows g(gate), v(as(saved[1], gate.scalar_type())), y(as(gr[0], gate.scalar_type()));
+    const Tensor &gate = saved[0], value = as(saved[1], gate.scalar_type()), dy = as(gr[0], gate.scalar_type());
+    need(gate, {{value, gate.sizes()}, {dy, gate.sizes()}});
+    const Rows g(gate), v(value), y(dy);
     const auto opt = gate.options().memory_format(at::MemoryFormat::Contiguous);
     Tensor dg = at::empty(gate.sizes(), opt), dv = at::empty(gate.sizes(), opt);
     check(kat_rswiglu_bwd(y.p(), g.p(), v.p(), dg.data_ptr(), dv.data_ptr(), g.rows, g.cols, y.ld, g.ld, v.ld, g.cols,
@@ -207,9 +218,11 @@ struct PackedSwiglu : Function<PackedSwiglu> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list gr) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor& gv = saved[0];
-    need(gv, {&gr[0]});
-    const Rows r(gv), y(as(gr[0], gv.scalar_type()));
+    const Tensor &gv = saved[0], dy = as(gr[0], gv.scalar_type());
+    auto half = gv.sizes().vec();
+    if (!half.empty()) half.back() /= 2;
+    need(gv, {{dy, half}});
+    const Rows r(gv), y(dy);
     const int64_t f = r.cols / 2, es = gv.element_size();
     Tensor d = at::empty(gv.sizes(), gv.options().memory_format(at::MemoryFormat::Contiguous));
     char *const g = (char*)r.p(), *const o = (char*)d.data_ptr();
@@ -231,6 +244,12 @@ bool weight_ok(const Tensor& x, const Tensor& w) {
          (w.scalar_type() == x.scalar_type() || (w.scalar_type() == at::kFloat && x.scalar_type() != at::kDouble));
 }
 
+// a saved weight in a dtype the kernels take
+Tensor saved_weight(const Tensor& x, const Tensor& w) {
+  const at::ScalarType xt = x.scalar_type(), wide = xt == at::kDouble ? at::kDouble : at::kFloat;
+  return as(w, w.scalar_type() == xt ? xt : wide).reshape({-1}).contiguous();
+}
+
 Tensor dw_like(const Tensor& x, int64_t cols) {
   return at::empty({cols}, x.options().dtype(x.scalar_type() == at::kDouble ? at::kDouble : at::kFloat));
 }
@@ -249,9 +268,10 @@ struct Norm : Function<Norm> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list gr) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &x = saved[0], w = saved[1].contiguous(), mean = saved[2].contiguous();
-    need(x, {&w, &mean, &gr[0]});
-    const Rows r(x), g(as(gr[0], x.scalar_type()));
+    const Tensor &x = saved[0], dy = as(gr[0], x.scalar_type());
+    const Rows r(x), g(dy);
+    const Tensor w = saved_weight(x, saved[1]), mean = as(saved[2], at::kFloat).contiguous();
+    need(x, {{w, {r.cols}}, {mean, {r.rows}}, {dy, x.sizes()}});
     Tensor dx = at::empty(x.sizes(), x.options().memory_format(at::MemoryFormat::Contiguous)), dw = dw_like(x, r.cols);
     const size_t wsb = kat_men_bwd_workspace_size(r.rows, r.cols, code(x));
     const Tensor ws = bytes(wsb, x);
@@ -281,16 +301,19 @@ struct AddNorm : Function<AddNorm> {
           "kat_add_men_fwd");
     ctx->save_for_backward({h, w, mean});
     ctx->saved_data["eps"] = eps;
+    ctx->saved_data["x"] = (int64_t)x.scalar_type();
     ctx->saved_data["r"] = (int64_t)r.scalar_type();
     ctx->saved_data["y"] = (int64_t)yt;
     return {h, y};
   }
   static variable_list backward(AutogradContext* ctx, variable_list gr) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &h = saved[0], w = saved[1].contiguous(), mean = saved[2].contiguous();
-    need(h, {&w, &mean, &gr[0], &gr[1]});
     const auto rt = (at::ScalarType)ctx->saved_data["r"].toInt(), yt = (at::ScalarType)ctx->saved_data["y"].toInt();
-    const Rows rh(h), g(as(gr[1], yt)), d(as(gr[0], h.scalar_type()));
+    const Tensor h = as(saved[0], (at::ScalarType)ctx->saved_data["x"].toInt());
+    const Tensor dy = as(gr[1], yt), dh = as(gr[0], h.scalar_type());
+    const Rows rh(h), g(dy), d(dh);
+    const Tensor w = saved_weight(h, saved[1]), mean = as(saved[2], at::kFloat).contiguous();
+    need(h, {{w, {rh.cols}}, {mean, {rh.rows}}, {dy, h.sizes()}, {dh, h.sizes()}});
     const auto opt = h.options().memory_format(at::MemoryFormat::Contiguous);
     Tensor dx = at::empty(h.sizes(), opt), dr, dw = dw_like(h, rh.cols);
     // a same-dtype branch gets the stream's gradient itself, a narrower one its cast
@@ -417,6 +440,11 @@ void python_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor&
                               km.defined() ? py::cast(km) : none, extended);
 }
 
+void need_dims(const Tensor& a, int64_t n) {
+  if (a.dim() != n || (n == 5 && a.size(2) != 3))
+    throw std::runtime_error("backward: a saved attention input has lost its dimensions");
+}
+
 // the key mask a backward unpacked (undefined: none) as the kernels read it:
 // uint8, rows of T bytes
 Tensor saved_mask(const Tensor& q, const Tensor& km, int64_t B, int64_t T) {
@@ -460,14 +488,16 @@ struct Attention : Function<Attention> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list gr) {
     const auto s = ctx->get_saved_variables();
-    need(s[0], {&s[1], &s[2], &s[3], &s[4], &s[5], &gr[0]});
     const at::ScalarType dt = s[0].scalar_type();
     const Tensor &q = s[0], k = as(s[1], dt), v = as(s[2], dt), o = as(s[3], dt), L = as(s[4], at::kFloat);
-    const Tensor &slopes = s[5], km = saved_mask(q, s[6], q.size(0), q.size(2));
+    Tensor go = as(gr[0], dt);
+    need_dims(q, 4);
+    const Tensor slopes = s[5].reshape({-1}), km = saved_mask(q, s[6], q.size(0), q.size(2));
+    need(q, {{k, q.sizes()}, {v, q.sizes()}, {o, q.sizes()}, {L, q.sizes().slice(0, 3)}, {slopes, {q.size(1)}},
+             {go, q.sizes()}});
     const double scale = ctx->saved_data["scale"].toDouble(), eps = ctx->saved_data["eps"].toDouble();
     const bool extended = ctx->saved_data["extended"].toBool(), causal = ctx->saved_data["causal"].toBool();
     const Dims n{q.size(0), q.size(1), q.size(2), q.size(3)};
-    Tensor go = as(gr[0], dt);
     if (go.stride(-1) != 1 && n.D != 1) go = go.contiguous();
     const auto opt = q.options().memory_format(at::MemoryFormat::Contiguous);
     Tensor dq = at::empty(q.sizes(), opt), dk = at::empty(q.sizes(), opt), dv = at::empty(q.sizes(), opt);
@@ -518,12 +548,14 @@ struct PackedAttention : Function<PackedAttention> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list gr) {
     const auto s = ctx->get_saved_variables();
-    need(s[0], {&s[1], &s[2], &s[3], &gr[0]});
-    const Tensor &qkv = s[0], y = as(s[1], qkv.scalar_type()), L = as(s[2], at::kFloat), &slopes = s[3];
+    const Tensor &qkv = s[0], y = as(s[1], qkv.scalar_type()), L = as(s[2], at::kFloat), slopes = s[3].reshape({-1});
+    Tensor go = as(gr[0], qkv.scalar_type());
+    need_dims(qkv, 5);
+    const int64_t yd[] = {qkv.size(0), qkv.size(1), qkv.size(3), qkv.size(4)}, ld[] = {yd[0], yd[2], yd[1]};
+    need(qkv, {{y, yd}, {L, ld}, {slopes, {yd[2]}}, {go, yd}});
     const Tensor km = saved_mask(qkv, s[4], qkv.size(0), qkv.size(1));
     const double scale = ctx->saved_data["scale"].toDouble(), eps = ctx->saved_data["eps"].toDouble();
     const Dims n{qkv.size(0), qkv.size(3), qkv.size(1), qkv.size(4)};
-    Tensor go = as(gr[0], qkv.scalar_type());
     if (go.stride(-1) != 1 && n.D != 1) go = go.contiguous();
     Tensor d = at::empty(qkv.sizes(), qkv.options().memory_format(at::MemoryFormat::Contiguous));
     if (qkv.stride(-1) == 1 && y.stride(-1) == 1 && go.stride(-1) == 1 && slopes_ok(qkv, slopes, n.H) &&

@@ -51,9 +51,10 @@ class RationalSoftmax(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         x, out = ctx.saved_tensors
+        _lib.need(x, (out, x.shape), (grad_output, x.shape))
         lib = _lib.load()
         x2, ldx = _lib.rows2d(x)
-        p2, ldp = _lib.rows2d(out)
+        p2, ldp = _lib.rows2d(out.to(x.dtype))
         g2, ldg = _lib.rows2d(grad_output.to(x.dtype))
         rows, cols = x2.shape
         dx = torch.empty((rows, cols), dtype=x.dtype, device=x.device)
@@ -85,9 +86,10 @@ class RationalSwiGLU(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         gate, value = ctx.saved_tensors
+        _lib.need(gate, (value, gate.shape), (grad_output, gate.shape))
         lib = _lib.load()
         g2, ldg = _lib.rows2d(gate)
-        v2, ldv = _lib.rows2d(value)
+        v2, ldv = _lib.rows2d(value.to(gate.dtype))
         y2, ldy = _lib.rows2d(grad_output.to(gate.dtype))
         rows, cols = g2.shape
         dgate = torch.empty((rows, cols), dtype=gate.dtype, device=gate.device)
@@ -126,6 +128,7 @@ class PackedRationalSwiGLU(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         (gv,) = ctx.saved_tensors
+        _lib.need(gv, (grad_output, (*gv.shape[:-1], gv.shape[-1] // 2)))
         lib = _lib.load()
         g2, ld = _lib.rows2d(gv)
         rows, two_f = g2.shape
@@ -174,6 +177,8 @@ class MeanErrorNorm(torch.autograd.Function):
         x2, ldx = _lib.rows2d(x)
         g2, ldg = _lib.rows2d(grad_output.to(x.dtype))
         rows, cols = x2.shape
+        w, mean = _weight_for(x, w).view(-1), mean.float().contiguous()
+        _lib.need(x, (w, (cols,)), (mean, (rows,)), (grad_output, x.shape))
         code = _lib.dtype_code(x)
         dx = torch.empty((rows, cols), dtype=x.dtype, device=x.device)
         acc = torch.float64 if x.dtype == torch.float64 else torch.float32
@@ -220,6 +225,7 @@ class ResidualMeanErrorNorm(torch.autograd.Function):
                                        _lib.dtype_code(w), _lib.stream(x)), "kat_add_men_fwd")
         ctx.save_for_backward(h, w, mean)
         ctx.eps = eps
+        ctx.h_dtype = h.dtype
         ctx.r_dtype = r.dtype
         ctx.y_dtype = y.dtype
         return h.view(x.shape), y.view(x.shape)
@@ -228,7 +234,11 @@ class ResidualMeanErrorNorm(torch.autograd.Function):
     def backward(ctx, grad_h, grad_y):
         h, w, mean = ctx.saved_tensors
         lib = _lib.load()
+        h = h.to(ctx.h_dtype).contiguous()
         rows, cols = h.shape
+        w, mean = _weight_for(h, w).view(-1), mean.float().contiguous()
+        _lib.need(h, (w, (cols,)), (mean, (rows,)), (h, (grad_y.numel() // cols if cols else rows, grad_y.shape[-1])),
+                  (grad_y, grad_h.shape), (grad_h, grad_h.shape))
         g2, ldg = _lib.rows2d(grad_y.to(ctx.y_dtype))
         d2, ldd = _lib.rows2d(grad_h.to(h.dtype))
         code = _lib.dtype_code(h)

@@ -244,6 +244,87 @@ def test_saved_key_mask_of_another_layout_or_place(gpu, D):
                 _plain_grads(fn, ins)
 
 
+def _class_ops():
+    x = _rand(1, 6, 64, dtype=torch.bfloat16)
+    w = torch.ones(64, device="cuda")
+    q = [_rand(i, 1, 2, 33, 64, dtype=torch.bfloat16) for i in range(3)]
+    slopes = F.compute_alibi_slopes(2).cuda()
+    return [("softmax class", lambda a: F.RationalSoftmax.apply(a, 1e-6), [x]),
+            ("swiglu class", F.RationalSwiGLU.apply, [x, x.clone()]),
+            ("packed swiglu class", F.PackedRationalSwiGLU.apply, [x]),
+            ("norm class", lambda a, b: F.MeanErrorNorm.apply(a, b, 1e-6), [x, w]),
+            ("add norm class", lambda a, b, c: F.ResidualMeanErrorNorm.apply(a, b, c, 1e-6, None)[1],
+             [x, x.clone(), w]),
+            ("attention class", lambda a, b, c: F.RationalAttentionFunction.apply(a, b, c, slopes, 0.125, True, 1e-6),
+             q)]
+
+
+def test_one_saved_tensor_of_another_layout_type_size_or_place(gpu):
+    """Each saved tensor alone comes back changed from a saved-tensor hook: in
+    a wider dtype and with a row stride it gives the same gradients (but for
+    the first, whose dtype is the launch's); with fewer rows or columns or on
+    the host it raises before any launch."""
+    def strided(t):
+        wide = torch.empty(t.shape[:-1] + (t.shape[-1] + 9,), dtype=torch.float64, device="cuda")
+        return wide[..., 1:t.shape[-1] + 1].copy_(t)
+
+    def one(i, change):
+        n = [0]
+
+        def pack(t):
+            n[0] += 1
+            return n[0] - 1, t
+        return torch.autograd.graph.saved_tensors_hooks(pack, lambda p: change(p[1]) if p[0] == i else p[1])
+
+    for name, fn, ins in _ops_list() + _class_ops() + _masked_ops(64):
+        saved = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: saved.append(t.dtype) or t, lambda t: t):
+            _, g0 = _plain_grads(fn, ins)
+        for i, dt in enumerate(saved):
+            if i > 0 and dt != torch.uint8:
+                with one(i, strided):
+                    _, g = _plain_grads(fn, ins)
+                assert all(torch.equal(a, b) for a, b in zip(g, g0)), (name, i)
+            for change in (lambda t: t[..., :-1], lambda t: t[:-1]):
+                with one(i, change), pytest.raises(RuntimeError):
+                    _plain_grads(fn, ins)
+            try:
+                with one(i, lambda t: t.cpu()):
+                    _, g = _plain_grads(fn, ins)
+            except (RuntimeError, AssertionError):
+                continue
+            # the classes move the slopes to the device, as their forward does
+            assert dt == torch.float32 and name.endswith("class"), (name, i)
+            assert all(torch.equal(a, b) for a, b in zip(g, g0)), (name, i)
+    # a probability saved narrower than its logits (fp32) is widened before it is read
+    x = _rand(3, 9, 65).requires_grad_(True)
+    for fn in (F.rational_softmax, lambda t: F.RationalSoftmax.apply(t, 1e-6)):
+        want = torch.autograd.grad(fn(x), x, _rand(4, 9, 65))[0]
+        with one(1, lambda t: t.bfloat16()):
+            got = torch.autograd.grad(fn(x), x, _rand(4, 9, 65))[0]
+        assert float((got - want).norm() / want.norm()) < 2.0 ** -7  # p's bf16 rounding, 2^-9 a factor
+
+
+def test_batched_gradients_raise(gpu):
+    for name, fn, ins in _ops_list() + _class_ops():
+        leaves = [t.detach().clone().requires_grad_(True) for t in ins]
+        y = fn(*leaves)
+        with pytest.raises(RuntimeError):
+            torch.autograd.grad(y, leaves, torch.ones(2, *y.shape, dtype=y.dtype, device="cuda"),
+                                is_grads_batched=True)
+
+
+def test_negated_gradient_views(gpu):
+    """A gradient that is a lazily negated view is read as its values."""
+    for name, fn, ins in _ops_list():
+        leaves = [t.detach().clone().requires_grad_(True) for t in ins]
+        y = fn(*leaves)
+        c = _rand(8, *y.shape, dtype=y.dtype)
+        want = torch.autograd.grad(y, leaves, -c, retain_graph=True)
+        got = torch.autograd.grad(y, leaves, torch._neg_view(c))
+        assert all(torch.equal(a, b) for a, b in zip(want, got)), name
+
+
 def test_modes_and_partial_gradients(gpu):
     for name, fn, ins in _ops_list():
         y0, g0 = _plain_grads(fn, ins)
