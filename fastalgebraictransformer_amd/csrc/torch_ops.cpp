@@ -381,6 +381,17 @@ bool attn_dtype(const Tensor& t) { return plain(t) && code(t) != KAT_F64; }
 bool slopes_ok(const Tensor& q, const Tensor& s, int64_t H) {
   return same_place(q, {&s}) && s.scalar_type() == at::kFloat && s.is_contiguous() && s.numel() == H;
 }
+// slopes of a module cast whole (bf16 / fp16, as its buffer becomes), which the
+// entry points convert as the Python functions do
+bool slopes_narrow(const Tensor& q, const Tensor& s, int64_t H) {
+  return same_place(q, {&s}) && (s.scalar_type() == at::kBFloat16 || s.scalar_type() == at::kHalf) &&
+         !s.requires_grad() && s.numel() == H;
+}
+Tensor slopes_of(const Tensor& s) {
+  if (s.scalar_type() == at::kFloat) return s;
+  at::NoGradGuard g;
+  return s.to(at::kFloat).contiguous();
+}
 
 struct Dims {
   int64_t B, H, T, D;
@@ -518,19 +529,19 @@ bool attn_ok(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& sl
          q.numel() > 0 && q.stride(3) == 1 && k.stride(3) == 1 && v.stride(3) == 1 &&
          head_dim_ok(q.size(3), q.element_size()) &&
          in_envelope({bhtd(q), bhtd(k), bhtd(v)}, q.size(2), q.size(3), q.element_size()) &&
-         slopes_ok(q, slopes, q.size(1));
+         (slopes_ok(q, slopes, q.size(1)) || slopes_narrow(q, slopes, q.size(1)));
 }
 
 std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& slopes, double scale,
                                 double eps) {
   if (!attn_ok(q, k, v, slopes)) return std::nullopt;
-  return Attention::apply(q, k, v, slopes, scale, eps, Mask{}, false, true);
+  return Attention::apply(q, k, v, slopes_of(slopes), scale, eps, Mask{}, false, true);
 }
 
 std::optional<Tensor> attention_masked(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& slopes,
                                        double scale, const std::optional<Tensor>& km, bool causal, double eps) {
   if (!attn_ok(q, k, v, slopes) || !mask_ok(q, km, q.size(0), q.size(2))) return std::nullopt;
-  return Attention::apply(q, k, v, slopes, scale, eps, mask_of(km), true, causal);
+  return Attention::apply(q, k, v, slopes_of(slopes), scale, eps, mask_of(km), true, causal);
 }
 
 struct PackedAttention : Function<PackedAttention> {
@@ -576,9 +587,10 @@ std::optional<Tensor> attention_packed(const Tensor& qkv, const Tensor& slopes, 
   if (!untraced() || !attn_dtype(qkv) || qkv.dim() != 5 || qkv.size(2) != 3 || qkv.numel() == 0 ||
       qkv.stride(4) != 1 || !head_dim_ok(qkv.size(4), qkv.element_size()) ||
       !in_envelope({part(qkv, 0), part(qkv, 1), part(qkv, 2)}, qkv.size(1), qkv.size(4), qkv.element_size()) ||
-      !slopes_ok(qkv, slopes, qkv.size(3)) || !mask_ok(qkv, km, qkv.size(0), qkv.size(1)))
+      !(slopes_ok(qkv, slopes, qkv.size(3)) || slopes_narrow(qkv, slopes, qkv.size(3))) ||
+      !mask_ok(qkv, km, qkv.size(0), qkv.size(1)))
     return std::nullopt;
-  return PackedAttention::apply(qkv, slopes, scale, eps, mask_of(km));
+  return PackedAttention::apply(qkv, slopes_of(slopes), scale, eps, mask_of(km));
 }
 
 // q [B, H, D] against caches [B, H, T, D]: (out, L); no gradient
@@ -588,7 +600,8 @@ std::optional<std::tuple<Tensor, Tensor>> decode(const Tensor& q, const Tensor& 
   if (!untraced() || !attn_dtype(q) || !same_place(q, {&k, &v}) || k.scalar_type() != q.scalar_type() ||
       v.scalar_type() != q.scalar_type() || q.dim() != 3 || k.dim() != 4 || k.sizes() != v.sizes() ||
       k.size(0) != q.size(0) || k.size(1) != q.size(1) || k.size(3) != q.size(2) || q.numel() == 0 ||
-      k.numel() == 0 || q.stride(2) != 1 || k.stride(3) != 1 || v.stride(3) != 1 || !slopes_ok(q, slopes, q.size(1)))
+      k.numel() == 0 || q.stride(2) != 1 || k.stride(3) != 1 || v.stride(3) != 1 ||
+      !(slopes_ok(q, slopes, q.size(1)) || slopes_narrow(q, slopes, q.size(1))))
     return std::nullopt;
   if (lengths && !(lengths->defined() && lengths->is_cuda() && lengths->device() == q.device() &&
                    lengths->layout() == at::kStrided && lengths->scalar_type() == at::kInt &&
@@ -596,6 +609,7 @@ std::optional<std::tuple<Tensor, Tensor>> decode(const Tensor& q, const Tensor& 
                    !lengths->key_set().has(c10::DispatchKey::Python)))
     return std::nullopt;
   at::NoGradGuard g;
+  const Tensor sl = slopes_of(slopes);
   const int64_t B = q.size(0), H = q.size(1), D = q.size(2), T = k.size(2);
   Tensor out = at::empty({B, H, D}, q.options().memory_format(at::MemoryFormat::Contiguous));
   Tensor L = at::empty({B, H}, q.options().dtype(at::kFloat));
@@ -604,7 +618,7 @@ std::optional<std::tuple<Tensor, Tensor>> decode(const Tensor& q, const Tensor& 
   const int64_t s[10] = {q.stride(0), q.stride(1), k.stride(0), k.stride(1), k.stride(2),
                          v.stride(0), v.stride(1), v.stride(2), out.stride(0), out.stride(1)};
   check(kat_attn_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), L.data_ptr<float>(),
-                        slopes.data_ptr<float>(), lengths ? lengths->data_ptr<int32_t>() : nullptr, ws.data_ptr(),
+                        sl.data_ptr<float>(), lengths ? lengths->data_ptr<int32_t>() : nullptr, ws.data_ptr(),
                         wsb, B, H, T, D, s, (float)scale, (float)eps, code(q), stream(q)),
         "kat_attn_decode");
   return std::make_tuple(out, L);

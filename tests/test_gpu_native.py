@@ -151,6 +151,37 @@ def test_decode(gpu):
         F.rational_attention_decode(q[..., :60], k[..., :60], v[..., :60], slopes, 0.125)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_slopes_of_a_model_cast_whole(gpu, dtype):
+    """A module cast whole holds 16-bit slopes: its attention, training and
+    decode, takes the native route with the classes' results."""
+    H, scale = 3, 0.125
+    slopes = F.compute_alibi_slopes(H).cuda().to(dtype)
+    q = [_rand(i, 2, H, 70, 64, dtype=dtype).requires_grad_(True) for i in range(3)]
+    km = torch.rand(2, 70, generator=torch.Generator().manual_seed(1)).cuda() > 0.3
+    ops = _lib.ops()
+    assert ops.attention(*q, slopes, scale, 1e-6) is not None
+    _same(lambda a, b, c: F.rational_attention(a, b, c, slopes, scale),
+          lambda a, b, c: F.RationalAttentionFunction.apply(a, b, c, slopes, scale, True, 1e-6), q, 5, "plain")
+    assert ops.attention_masked(*q, slopes, scale, km, False, 1e-6) is not None
+    _same(lambda a, b, c: F.rational_attention_masked(a, b, c, slopes, scale, km, False),
+          lambda a, b, c: F.backward.MaskedRationalAttentionFunction.apply(a, b, c, slopes, scale, km, False, 1e-6),
+          q, 5, "masked")
+    p = _rand(4, 2, 70, 3, H, 64, dtype=dtype).requires_grad_(True)
+    assert ops.attention_packed(p, slopes, scale, 1e-6, None) is not None
+    _same(lambda t: F.rational_attention_packed(t, slopes, scale),
+          lambda t: F.PackedRationalAttention.apply(t, slopes, scale, 1e-6, None), [p], 5, "packed")
+    one = q[0][:, :, 0].detach()
+    assert ops.decode(one, q[1], q[2], slopes, scale, None, 1e-6) is not None
+    # the Python route: the same slopes in a dtype the native functions leave to it
+    for a, b in zip(F.rational_attention_decode(one, q[1], q[2], slopes, scale),
+                    F.rational_attention_decode(one, q[1], q[2], slopes.double(), scale)):
+        assert torch.equal(a, b)
+    # slopes that ask for a gradient, or of the wrong count, stay with the classes
+    assert ops.attention(*q, slopes.clone().requires_grad_(True), scale, 1e-6) is None
+    assert ops.attention(*q, slopes[:2], scale, 1e-6) is None
+
+
 def _ops_list():
     x = _rand(1, 6, 64, dtype=torch.bfloat16)
     w = torch.ones(64, device="cuda")
