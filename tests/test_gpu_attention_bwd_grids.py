@@ -57,21 +57,25 @@ def test_both_sides_of_the_dispatch(gpu, D, H, T, causal):
     _case(1, H, T, D, torch.bfloat16, causal=causal)
 
 
-@pytest.mark.parametrize("H", [1, 4, 12, 17])
-def test_head_groups_of_any_head_count(gpu, H, monkeypatch):
-    """One group of all heads (they fit) against groups of one head each: the
-    same bits, and a workspace that the size query covers."""
+# (heads, heads that the capped workspace holds, heads of a group then: capped
+# groups of 8 or more are rounded down to a multiple of 8)
+@pytest.mark.parametrize("H,fit,group", [(1, 1, 1), (4, 1, 1), (12, 1, 1), (12, 10, 8), (17, 10, 8), (17, 16, 16)])
+def test_head_groups_of_any_head_count(gpu, H, fit, group, monkeypatch):
+    """One group of all heads (they fit) against capped groups: the same bits,
+    and a workspace that shrinks to the group's."""
     T, D = 300, 64
+    head = 40 * 8192  # dS^T of a head at T = 300: 5 key tiles of 8 query tiles, 8 KB each
     lib = _lib.load()
     g = torch.Generator().manual_seed(H)
     q, k, v, do = (torch.randn(1, H, T, D, generator=g).to(torch.bfloat16).to(dev) for _ in range(4))
     slopes = F.compute_alibi_slopes(H).to(dev)
     o, L = F.rational_attention_forward(q, k, v, slopes, 0.125)
-    got = []
-    for cap in (None, 1):
+    got, ws = [], []
+    for cap in (None, fit * head):
         if cap:
-            monkeypatch.setenv("KAT_ATTN_DS_CAP_BYTES", str(200 * 8192))  # ~5 of the 15 tiles' heads at T = 300
-        assert lib.kat_attn_bwd_workspace_size(1, H, T, D, 1) > 0
+            monkeypatch.setenv("KAT_ATTN_DS_CAP_BYTES", str(cap))
+        ws.append(lib.kat_attn_bwd_workspace_size(1, H, T, D, 1))
         got.append(F.rational_attention_backward(q, k, v, o, L, do, slopes, 0.125))
+    assert ws[0] - ws[1] == (H - group) * head
     for a, b in zip(*got):
         assert torch.equal(a, b)
