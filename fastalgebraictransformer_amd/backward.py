@@ -26,6 +26,12 @@ from .forward import (  # noqa: F401
 )
 
 
+def _need_saved(q, k, v, output, L, grad_output):
+    """What a class's backward unpacked and was handed, as [B, H, T, D] tensors
+    and L [B, H, T], before the launch reads them."""
+    _lib.need(q, (k, q.shape), (v, q.shape), (output, q.shape), (grad_output, q.shape), (L, q.shape[:3]))
+
+
 def _attn_bwd_into(q, k, v, output, L, grad_output, dq, dk, dv, alibi_slopes, scale, causal, eps,
                    key_mask=None, extended=False):
     """Launch the attention backward; every [B,H,T,D] argument may have any
@@ -38,8 +44,6 @@ def _attn_bwd_into(q, k, v, output, L, grad_output, dq, dk, dv, alibi_slopes, sc
     q = _unit_d(q)
     k, v, output, grad_output = (_unit_d(t.to(q.dtype)) for t in (k, v, output, grad_output))
     L = L.to(torch.float32)
-    _lib.need(q, (k, q.shape), (v, q.shape), (output, q.shape), (grad_output, q.shape),
-              (L, (B, H, T) + L.shape[3:]))
     if key_mask is not None:  # saved by the forward as uint8 [B, T]; a hook may return it otherwise
         if key_mask.device != q.device or key_mask.dtype != torch.uint8 or key_mask.shape != (B, T):
             raise RuntimeError("backward: the saved key mask must be uint8 [B, T] on the inputs' device")
@@ -106,6 +110,7 @@ class RationalAttentionFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         q, k, v, output, L, alibi_slopes = ctx.saved_tensors
+        _need_saved(q, k, v, output, L, grad_output)
         dq, dk, dv = rational_attention_backward(q, k, v, output, L, grad_output, alibi_slopes,
                                                  ctx.scale, ctx.causal, ctx.eps)
         return dq, dk, dv, None, None, None, None
@@ -147,7 +152,8 @@ class PackedRationalAttention(torch.autograd.Function):
     def backward(ctx, grad_y):
         qkv, y, L, alibi_slopes, km = ctx.saved_tensors
         q, k, v = qkv.permute(2, 0, 3, 1, 4)
-        grad_o = _unit_d(grad_y.to(qkv.dtype).permute(0, 2, 1, 3))
+        grad_o = grad_y.permute(0, 2, 1, 3)
+        _need_saved(q, k, v, y.permute(0, 2, 1, 3), L, grad_o)
         dqkv = torch.empty(qkv.shape, dtype=qkv.dtype, device=qkv.device)
         dq, dk, dv = dqkv.permute(2, 0, 3, 1, 4)
         _attn_bwd_into(q, k, v, y.permute(0, 2, 1, 3), L, grad_o, dq, dk, dv, alibi_slopes,
@@ -188,9 +194,9 @@ class MaskedRationalAttentionFunction(torch.autograd.Function):
     def backward(ctx, grad_output):
         q, k, v, out, L, alibi_slopes, km = ctx.saved_tensors
         B, H, T, D = q.shape
-        go = _unit_d(grad_output.to(q.dtype))
+        _need_saved(q, k, v, out, L, grad_output)
         dq, dk, dv = (torch.empty((B, H, T, D), dtype=q.dtype, device=q.device) for _ in range(3))
-        _attn_bwd_into(q, k, v, out, L, go, dq, dk, dv, alibi_slopes, ctx.scale, ctx.causal,
+        _attn_bwd_into(q, k, v, out, L, grad_output, dq, dk, dv, alibi_slopes, ctx.scale, ctx.causal,
                        ctx.eps, km, extended=True)
         return dq, dk, dv, None, None, None, None, None
 
