@@ -1025,17 +1025,25 @@ template <typename A> __global__ void fill_zero_k(A* __restrict__ p, int64_t n) 
 // Host launchers
 // ============================================================================
 
-// Persistent row grids: up to `per_cu` 256-thread blocks per compute unit. With
+// Persistent row grids: up to 8 256-thread blocks per compute unit. With
 // many rows a block takes at least 4, so that the two-row prefetch (which
 // clamps past the last row) wastes little; with few it takes 2 or 1, since the
 // rows of a block run one after the other (norm forward, one row per block
 // against 4: 8 x 4096 bf16 4.3 -> 2.3 us, 256 x 4096 5.4 -> 3.5, 512 x 2048
-// residual 7.4 -> 5.4; two: 2048 x 4096 11.3 -> 10.2; from 4096 rows on 4).
+// residual 7.4 -> 5.4). `held` says how much of a row a thread holds (chunk rounds
+// times streams: residual norm and softmax backward 2): the more, the fewer blocks
+// a CU keeps resident, and the sooner fewer rows per block only lengthen
+// the tail. Measured, us, 2 rows per block / 4: held 1-2: norm bf16 2048 x 4096
+// 10.2 / 11.3, 1536 x 2304 at 0.85 of it; 4-8: residual bf16 1024 x 6144 0.85,
+// 2047 x 8192 33.0 / 30.4, softmax backward bf16 1280 x 8192 0.89, 2047 x 8192
+// 31.3 / 29.5; above: softmax backward bf16 400 x 16384 0.69 (1 row: 0.81),
+// 640 x 16384 1.21, 2047 x 16384 75.6 / 63.0, fp32 2047 x 8192 75.8 / 63.2.
 constexpr int kRowBlocksPerCU = 8;
-static inline int64_t row_grid(int64_t rows, int per_cu) {
+static inline int64_t row_grid(int64_t rows, int held) {
   const int64_t cus = num_cus();
-  const int64_t per = rows <= 2 * cus ? 1 : rows <= 8 * cus ? 2 : 4;
-  return std::max<int64_t>(1, std::min<int64_t>((int64_t)per_cu * cus, (rows + per - 1) / per));
+  const int64_t one = held <= 8 ? 2 : 1, two = held <= 2 ? 8 : held <= 8 ? 6 : 2;  // rows per CU up to which
+  const int64_t per = rows <= one * cus ? 1 : rows <= two * cus ? 2 : 4;
+  return std::max<int64_t>(1, std::min<int64_t>(kRowBlocksPerCU * cus, (rows + per - 1) / per));
 }
 
 // grid of the one-block-per-row kernels, which walk rows with a grid stride
@@ -1190,7 +1198,7 @@ static int rsoftmax_fwd_t(const T* x, T* p, int64_t rows, int64_t cols, int64_t 
     KAT_NCH_SWITCH8(nchw, hipLaunchKernelGGL((rsoftmax_fwd_w_k<T, N>), dim3(blocks), dim3(256), 0, st,
                                             x, p, rows, (int)cols, ldx, ldp, eps));
   } else if (nch) {
-    const int64_t blocks = row_grid(rows, kRowBlocksPerCU);
+    const int64_t blocks = row_grid(rows, nch);
     KAT_NCH_SWITCH(nch, hipLaunchKernelGGL((rsoftmax_fwd_k<T, N>), dim3((unsigned)blocks),
                                            dim3(256), 0, st, x, p, rows, (int)cols, ldx, ldp, eps));
   } else {
@@ -1215,7 +1223,7 @@ static int rsoftmax_bwd_t(const T* dy, const T* x, const T* p, T* dx, int64_t ro
                                             dy, x, p, dx, rows, (int)cols, lddy, ldx, ldp, lddx,
                                             eps));
   } else if (nch) {
-    const int64_t blocks = row_grid(rows, kRowBlocksPerCU);
+    const int64_t blocks = row_grid(rows, 2 * nch);
     KAT_NCH_SWITCH(nch, hipLaunchKernelGGL((rsoftmax_bwd_k<T, N>), dim3((unsigned)blocks),
                                            dim3(256), 0, st, dy, x, p, dx, rows, (int)cols, lddy,
                                            ldx, ldp, lddx, eps));
@@ -1246,7 +1254,7 @@ static int men_fwd_t(const T* x, const W* w, Y* y, float* mu, int64_t rows, int6
                            dim3(256), 0, st, x, w, y, mu, rows, (int)cols, ldx, ldy, eps,
                            (const void*)r, h, ldr, ldh));
   } else if (nch) {
-    const int64_t blocks = row_grid(rows, kRowBlocksPerCU);
+    const int64_t blocks = row_grid(rows, kAdd ? 2 * nch : nch);
     const bool full = cols == (int64_t)nch * 256 * V;
     KAT_NCH_SWITCH(nch, {
       if (kat_full_variant(N, full))
