@@ -1275,17 +1275,22 @@ static int men_fwd_t(const T* x, const W* w, Y* y, float* mu, int64_t rows, int6
 
 // Backward blocks. The dgamma partials cost G x cols x 4 bytes of extra traffic
 // (written here, read by colsum_k), so G is two blocks per CU at most, one per
-// CU below 16 rows per CU (2048 x 2048 15.5 -> 12.9 us) and for waves that hold
+// CU with few rows per CU and for waves that hold
 // 3 or 4 rounds of a row (16384 x 2048 46.4 -> 41.4; at 2 rounds, 16384 x 768,
 // one per CU is slower, 23.6 -> 30.0). Few rows: one or two per block, since a
 // block's rows run one after the other (8 x 768 7.2 -> 5.0, 512 x 2048
 // residual 10.6 -> 9.8). nchw: wave_norm_nch (0: a block per row).
-static int men_bwd_grid(int64_t rows, int nchw) {
+// The line of one block per CU depends on the row's bytes: rows that little more
+// than fill one chunk round leave most of the second idle and want the second
+// block sooner (one / two per CU: bf16 2048 x 2304 1.10, 3000 x 2056 23.0 / 20.1,
+// 3500 x 4096 1.07; 2048 x 4096 0.88, 3500 x 8192 0.85, fp32 3500 x 4096 0.95).
+static int men_bwd_grid(int64_t rows, int nchw, int64_t row_bytes) {
   const int64_t cus = num_cus();
   if (nchw) return (int)std::min<int64_t>((rows + 2 * kRowWaves - 1) / (2 * kRowWaves), (nchw <= 2 ? 2 : 1) * cus);
   if (2 * rows <= cus) return (int)std::max<int64_t>(1, rows);
   if (rows <= 2 * cus) return (int)((rows + 1) / 2);
-  return (int)(rows < 16 * cus ? std::min<int64_t>((rows + 3) / 4, cus) : 2 * cus);
+  const int64_t one = row_bytes >= 12288 ? 16 : row_bytes >= 8192 ? 10 : 6;  // rows per CU below which
+  return (int)std::min<int64_t>((rows + 3) / 4, (rows < one * cus ? 1 : 2) * cus);
 }
 
 template <typename T, typename W, typename R = void, typename Y = T>
@@ -1306,7 +1311,7 @@ static int men_bwd_t(const Y* dy, const T* x, const W* w, const float* mu, T* dx
           (dr == nullptr || (lddr % V == 0 && reinterpret_cast<uintptr_t>(dr) % (V * sizeof(R)) == 0));
   const int nch = vec ? pick_nch(cols, 256 * V) : 0;
   const int nchw = vec ? wave_norm_nch(rows, cols, V) : 0;
-  const int G = men_bwd_grid(rows, nchw);
+  const int G = men_bwd_grid(rows, nchw, cols * (int64_t)sizeof(T));
   const size_t need = (size_t)G * (size_t)cols * sizeof(A);
   if (ws_bytes < need || (need && ws == nullptr))
     return fail(KAT_EINVAL, "%s: workspace %zu bytes < required %zu", nm, ws_bytes, need);
@@ -1451,7 +1456,8 @@ extern "C" size_t kat_men_bwd_workspace_size(int64_t n_rows, int64_t n_cols, int
   const int sz = dtype_size(dtype);
   if (n_rows <= 0 || n_cols <= 0 || sz == 0) return 0;
   // alignment decides between the kernels at call time: size for the larger grid
-  const int G = std::max(men_bwd_grid(n_rows, 0), men_bwd_grid(n_rows, wave_norm_nch(n_rows, n_cols, 16 / sz)));
+  const int G = std::max(men_bwd_grid(n_rows, 0, n_cols * sz),
+                         men_bwd_grid(n_rows, wave_norm_nch(n_rows, n_cols, 16 / sz), n_cols * sz));
   const size_t acc = dtype == KAT_F64 ? 8 : 4;
   return (size_t)G * (size_t)n_cols * acc;
 }
