@@ -1105,6 +1105,17 @@ static inline int wave_norm_nch(int64_t rows, int64_t n_cols, int V) {
   const int64_t need = (n_cols + 64 * V - 1) / (64 * V);
   return rows > num_cus() && need <= 4 ? (int)need : 0;
 }
+// The same for the forward, where rows that fill four rounds go back to the block
+// kernels (which they fill too) between 28 and 64 rows per CU. Block / wave, of
+// the block's time, at 8192, 12000 and 16384 rows: norm bf16 x 2048 1.07, 1.03, 1.04,
+// fp32 x 1024 1.06, 1.09, 1.03, residual bf16 x 2048 1.09, 1.05, 1.00, of an fp32
+// stream x 1024 1.02, 1.01, 1.01; at 7000 0.99, 0.95, 1.11, 1.03, at 24000 1.02,
+// 1.03, 0.97, 0.98. The plain and the residual norm take the same line: they
+// sum a row in the same order, to the same bits.
+static inline int wave_fwd_nch(int64_t rows, int64_t n_cols, int V) {
+  const int64_t cus = num_cus();
+  return n_cols == 256 * V && rows > 28 * cus && rows <= 64 * cus ? 0 : wave_norm_nch(rows, n_cols, V);
+}
 // Forward blocks of 4 such rows: as many per CU as the registers of their two
 // prefetched rows keep resident (8 per CU: 16384 x 1024 residual 39.5 us
 // against 37.1 with 4, 4096 x 1024 fp32 11.0 against 8.8 with 2).
@@ -1246,7 +1257,7 @@ static int men_fwd_t(const T* x, const W* w, Y* y, float* mu, int64_t rows, int6
     vec = vec && ldr % V == 0 && ldh % V == 0 && aligned16(h) &&
           reinterpret_cast<uintptr_t>(r) % (V * sizeof(R)) == 0;
   const int nch = vec ? pick_nch(cols, 256 * V) : 0;
-  const int nchw = vec ? wave_norm_nch(rows, cols, V) : 0;
+  const int nchw = vec ? wave_fwd_nch(rows, cols, V) : 0;
   if (nchw) {
     const int64_t blocks = wave_row_grid(rows, nchw);
     const bool full = cols == (int64_t)nchw * 64 * V;
