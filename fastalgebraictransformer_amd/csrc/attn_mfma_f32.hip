@@ -730,24 +730,40 @@ int f32_width(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256
 // 365; 8 x 16 x 128 (256) 9.1 / 8.1 / 10.4; 16 x 12 x 128 (384) 11.6 / 13.0 / 14.7;
 // D = 128: 2 x 12 x 512 (192) 41.7 / 30.7; D = 32: 16.4 / 11.5; non-causal D = 64:
 // 2 x 16 x 512 (256) 25.0 / 24.0 / 27.2; 1 x 12 x 1024 (192) 45.7 / 43.1 / 38.7.
-int f32_fwd_groups(int D, bool causal, int64_t nb, int64_t T) {
+// Non-causal blocks are equal, so a split gains only where it fills idle CUs
+// (2 x 10 x 1024 (320) 81.3 / 69.8; 2 x 24 x 512, D = 128 (384) 0.88 of one group's
+// time), not past 1.5 blocks per CU (2 x 16 x 1024 (512) 82.6 / 87.5, D = 128 152 /
+// 162, 2 x 48 x 512 (768), D = 32 with padding 34 / 43), except that D = 32 gains
+// up to two (2 x 8 x 1024 (256) 0.93, 2 x 8 x 2048 (512) 0.98), nor in short sequences
+// (2 x 50 x 256, D = 128 (400) 43 / 48; 2 x 125 x 64, D = 128 (250) 11.1 / 12.9, causal
+// D = 64 7.3 / 8.1). A padding mask skips tiles, of which four groups gain nothing
+// (2 x 12 x 512 (192) 26.6 / 25.8 / 28.6). Causal D = 64 of up to 512 keys takes one
+// group from two blocks per CU on (2 x 48 x 512 (768) 39.0 / 42.9 with padding).
+int f32_fwd_groups(int D, bool causal, bool masked, int64_t nb, int64_t T) {
   const int64_t cus = num_cus();
   if (D > 128) return 1;
-  if (D == 64 && (2 * nb <= cus || (T > 256 && (causal ? nb <= cus : 4 * nb <= 3 * cus)))) return 4;
-  return nb <= cus || (T > 128 && nb <= 3 * cus) ? 2 : 1;
+  if (2 * nb <= cus) return D == 64 ? 4 : 2;
+  if (causal) {
+    if (T <= 64 || nb > (T <= 128 ? 1 : D == 64 && T <= 512 ? 2 : 3) * cus) return 1;
+    return D == 64 && T > 256 && nb <= cus ? 4 : 2;
+  }
+  if (D == 32 ? T <= 128 || nb > 2 * cus : T <= 256 || 2 * nb > 3 * cus) return 1;
+  return D == 64 && !masked && 4 * nb <= 3 * cus ? 4 : 2;
 }
 // The same for the backward's two kinds of blocks (nb of each). D = 64: 2 x 12 x 512
 // (192) 62.5 / 40.4 / 43.6; 1 x 10 x 1024 (160) 104 / 66 / 60; 1 x 8 x 1024 (128)
 // 86.4 / 70.2 / 47.4; 1 x 20 x 1024 (320) 121 / 105 / 108; 8 x 12 x 256 (384) 43.8 /
 // 46.1 / 53.9; 2 x 12 x 1024 (384) 120 / 121 / 128; D = 128: 1 x 12 x 1024 (192)
 // 213 / 117; D = 32: 2 x 12 x 512 (192) 38 / 27; non-causal: D = 64, 1 x 12 x 1024
-// (192) 130 / 111 / 112, D = 128, 1 x 16 x 1024 (256) 245 / 250.
-int f32_bwd_groups(int D, bool causal, int64_t nb) {
+// (192) 130 / 111 / 112, D = 128, 1 x 16 x 1024 (256) 245 / 250. Short sequences: 2 x 50
+// x 64 (100) 12.8 / 12.6 / 15.6, 2 x 20 x 256 (160) 34.6 / 24.7 / 28.6, 2 x 125 x 64
+// (250) 20.0 / 22.3.
+int f32_bwd_groups(int D, bool causal, int64_t nb, int64_t T) {
   const int64_t cus = num_cus();
   if (D > 128) return 1;
   if (!causal) return 4 * nb <= 3 * cus ? 2 : 1;
-  if (D == 64 && 8 * nb <= 5 * cus) return 4;
-  return nb <= cus ? 2 : 1;
+  if (D == 64 && T > 256 && 8 * nb <= 5 * cus) return 4;
+  return (T <= 64 ? 2 : 1) * nb <= cus ? 2 : 1;
 }
 
 template <int D, int MODE, int KG> int launch_fwd_f32_kg(const AttnArgs& a, hipStream_t st) {
@@ -757,7 +773,8 @@ template <int D, int MODE, int KG> int launch_fwd_f32_kg(const AttnArgs& a, hipS
   return check_launch("kat_attn_fwd (fp32 mfma)");
 }
 template <int D, int MODE> int launch_fwd_f32(const AttnArgs& a, hipStream_t st) {
-  const int kg = f32_fwd_groups(D, (MODE & kModeCausalF) != 0, (int64_t)((a.T + kF32BM - 1) / kF32BM) * a.B * a.H, a.T);
+  const int kg = f32_fwd_groups(D, (MODE & kModeCausalF) != 0, (MODE & kModeKeyMaskF) != 0,
+                                (int64_t)((a.T + kF32BM - 1) / kF32BM) * a.B * a.H, a.T);
   if constexpr (D == 64)
     if (kg == 4) return launch_fwd_f32_kg<D, MODE, 4>(a, st);
   if constexpr (D <= 128)
@@ -777,7 +794,7 @@ int launch_bwd_f32_kg(const AttnArgs& a, const float* delta, const float* cinv, 
 }
 template <int D, int MODE>
 int launch_bwd_f32(const AttnArgs& a, const float* delta, const float* cinv, hipStream_t st) {
-  const int kg = f32_bwd_groups(D, (MODE & kModeCausalF) != 0, (int64_t)((a.T + kF32BM - 1) / kF32BM) * a.B * a.H);
+  const int kg = f32_bwd_groups(D, (MODE & kModeCausalF) != 0, (int64_t)((a.T + kF32BM - 1) / kF32BM) * a.B * a.H, a.T);
   if constexpr (D == 64 && (MODE & kModeCausalF) != 0)
     if (kg == 4) return launch_bwd_f32_kg<D, MODE, 4>(a, delta, cinv, st);
   if constexpr (D <= 128)

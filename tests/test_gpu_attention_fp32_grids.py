@@ -55,12 +55,18 @@ def test_edges(gpu, D, T, mode):
     _case(1, 3, T, D, mode)
 
 
-# nb = H blocks of 64 rows (T <= 64) or 2 H; lines at 128, 160, 192, 256 and 768 blocks
+# nb = H ceil(T / 64) blocks of 64 rows; lines at 128, 160, 192, 256, 384, 512 and 768 blocks
+# and T = 64, 128, 256 and 512
 @pytest.mark.parametrize("D,H,T,mode", [
     (64, 128, 60, "causal"), (64, 129, 60, "causal"), (64, 160, 60, "causal"), (64, 161, 60, "causal"),
     (64, 256, 60, "causal"), (64, 257, 60, "causal"), (64, 51, 270, "causal"), (64, 52, 270, "causal"),
     (64, 256, 130, "causal"), (64, 257, 130, "causal"), (64, 192, 60, "noncausal"), (64, 193, 60, "noncausal"),
     (128, 256, 40, "causal"), (128, 257, 40, "causal"), (32, 256, 40, "causal"), (32, 257, 40, "masked"),
+    (128, 128, 64, "causal"), (128, 129, 64, "causal"), (128, 128, 65, "causal"), (32, 129, 64, "masked"),
+    (64, 170, 130, "causal"), (64, 171, 130, "causal"), (64, 76, 600, "causal"), (64, 77, 600, "masked"),
+    (64, 32, 270, "causal"), (64, 33, 270, "causal"), (32, 170, 130, "noncausal"), (32, 171, 130, "noncausal"),
+    (64, 38, 270, "noncausal"), (64, 39, 270, "noncausal"), (64, 76, 270, "noncausal"),
+    (64, 77, 270, "noncausal"), (128, 76, 270, "noncausal"), (128, 77, 270, "noncausal"),
 ])
 def test_both_sides_of_the_dispatch(gpu, D, H, T, mode):
     _case(1, H, T, D, mode)
