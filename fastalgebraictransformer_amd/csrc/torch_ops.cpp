@@ -137,6 +137,10 @@ Tensor as(const Tensor& t, at::ScalarType dt) {
   return r.scalar_type() == dt ? r : r.to(dt);
 }
 
+// a weight or slopes tensor, which may come with leading dims of 1 (a view op costs
+// a microsecond of host time)
+Tensor flat(const Tensor& t) { return t.dim() == 1 ? t : t.reshape({-1}); }
+
 Tensor bytes(size_t n, const Tensor& like) {
   return at::empty({(int64_t)std::max<size_t>(n, 1)}, like.options().dtype(at::kByte));
 }
@@ -247,7 +251,7 @@ bool weight_ok(const Tensor& x, const Tensor& w) {
 // a saved weight in a dtype the kernels take
 Tensor saved_weight(const Tensor& x, const Tensor& w) {
   const at::ScalarType xt = x.scalar_type(), wide = xt == at::kDouble ? at::kDouble : at::kFloat;
-  return as(w, w.scalar_type() == xt ? xt : wide).reshape({-1}).contiguous();
+  return flat(as(w, w.scalar_type() == xt ? xt : wide)).contiguous();
 }
 
 Tensor dw_like(const Tensor& x, int64_t cols) {
@@ -503,7 +507,7 @@ struct Attention : Function<Attention> {
     const Tensor &q = s[0], k = as(s[1], dt), v = as(s[2], dt), o = as(s[3], dt), L = as(s[4], at::kFloat);
     Tensor go = as(gr[0], dt);
     need_dims(q, 4);
-    const Tensor slopes = s[5].reshape({-1}), km = saved_mask(q, s[6], q.size(0), q.size(2));
+    const Tensor slopes = flat(s[5]), km = saved_mask(q, s[6], q.size(0), q.size(2));
     need(q, {{k, q.sizes()}, {v, q.sizes()}, {o, q.sizes()}, {L, q.sizes().slice(0, 3)}, {slopes, {q.size(1)}},
              {go, q.sizes()}});
     const double scale = ctx->saved_data["scale"].toDouble(), eps = ctx->saved_data["eps"].toDouble();
@@ -559,7 +563,7 @@ struct PackedAttention : Function<PackedAttention> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list gr) {
     const auto s = ctx->get_saved_variables();
-    const Tensor &qkv = s[0], y = as(s[1], qkv.scalar_type()), L = as(s[2], at::kFloat), slopes = s[3].reshape({-1});
+    const Tensor &qkv = s[0], y = as(s[1], qkv.scalar_type()), L = as(s[2], at::kFloat), slopes = flat(s[3]);
     Tensor go = as(gr[0], qkv.scalar_type());
     need_dims(qkv, 5);
     const int64_t yd[] = {qkv.size(0), qkv.size(1), qkv.size(3), qkv.size(4)}, ld[] = {yd[0], yd[2], yd[1]};
