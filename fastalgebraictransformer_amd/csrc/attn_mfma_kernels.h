@@ -617,11 +617,11 @@ __global__ __launch_bounds__(256) void attn_bwd_stscale_k(BwdWs ws, int T, int c
 // ============================================================================
 // dS^T tiles. The dK / dV kernel stores the fp16 dS it feeds its dK product
 // (2^kq dS, zero where a key is masked or past its query) for every 64-key x
-// 64-query tile (kt, qt) the backward touches, 8 KB each. Tiles are grouped by
-// the dQ kernel's blocks of kQB query tiles so that each dQ block streams one
-// contiguous run: a head's runs follow each other by query block qb, and
-// within a run come, key tile by key tile (kt = 0 .. the block's last, causal;
-// every kt otherwise), the block's kQB query tiles side by side (in causal
+// 64-query tile (kt, qt) the backward touches, 8 KB each. Tiles are grouped
+// into runs of kQB query tiles, of which a dQ block streams one whole or half (its
+// queries' columns): a head's runs follow each other by query block qb, and
+// within a run come, key tile by key tile (kt = 0 .. the run's last, causal;
+// every kt otherwise), the run's kQB query tiles side by side (in causal
 // mode the tiles with kt > qt inside a run are not written and not read).
 // Long sequences whose tiles exceed the workspace's cap run in bands of key
 // tiles [kb0, kb0 + nk) (kb0 and nk multiples of kQB, the last band shorter):
@@ -639,7 +639,7 @@ __global__ __launch_bounds__(256) void attn_bwd_stscale_k(BwdWs ws, int T, int c
 // backward). A 32-key half (one dQ stage) is the tile's first or second
 // contiguous 4 KB, which the dQ kernel's DMA permutes back into row order.
 // ============================================================================
-constexpr int kQB = 8;  // 64-query tiles per dQ block
+constexpr int kQB = 8;  // 64-query tiles per run
 
 // first tile of query block qb's run in the band [kb0, kb0 + nk): causal runs
 // hold min(nk, kQB (qb + 1) - kb0) key tiles (the last run: nk), the others nk
@@ -660,11 +660,14 @@ __device__ __forceinline__ int64_t ds_tile(int kt, int qt, bool causal, int kb0,
 __device__ __forceinline__ int ds_col_query(int c) { return 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3); }
 
 // ============================================================================
-// dQ from the stored dS: 512 queries (kQB 64-query tiles) per block, 8 waves,
-// each owning one 64-query tile, one block per CU; per 32-key half of a key
-// tile
+// dQ from the stored dS: 8 waves of QW queries per block; per 32-key half of a
+// key tile
 //   dQ^T[d][q] += K16^T[d][key] dS^T[key][q]   A = K16^T (LDS transposed)
 //                                              B = dS^T  (LDS transposed)
+// QW = 64: a wave owns a 64-query tile and the block a whole run of dS (512
+// queries; one block per CU). QW = 32: half a tile and half a run (256 queries),
+// at D = 256 (whose accumulators for 64 queries would take all 256 VGPRs) and
+// for grids short of the chip (bwd_small_dq).
 // A plain GEMM, bound by streaming the stored dS once. Each wave stages its
 // own dS rows (from the block's contiguous run, non-temporal LDS-DMA) and the
 // block shares the K rows, 32 keys per stage, four stages deep (two in flight
@@ -676,7 +679,7 @@ __device__ __forceinline__ int ds_col_query(int c) { return 16 * ((c >> 2) & 1) 
 // the dK/dV kernel formed for the same 32 keys (ek: its exponent, read from
 // kexp; the conversion is the same function, so K16 is bit-identical): the
 // backward keeps no fp16 copy of K in HBM, and this kernel's spare VALU does
-// the conversion. Each K16 fragment read from LDS feeds four MFMAs. Blocks
+// the conversion. Each K16 fragment read from LDS feeds QW / 16 MFMAs. Blocks
 // take the forward's order (heads pinned to XCDs, longest blocks first across
 // the XCD's heads). dS carries its query tile's 2^kq and K16 its 32 keys'
 // 2^ek: the accumulators are rescaled when ek changes and the epilogue
@@ -689,9 +692,7 @@ __device__ __forceinline__ int ds_col_query(int c) { return 16 * ((c >> 2) & 1) 
 // ============================================================================
 constexpr int kDqW = kQB;           // waves per dQ block
 constexpr int kDqS = 4;             // stages (32 keys each)
-// queries per dQ wave: a 64-query tile, or at D = 256 (whose accumulators for
-// 64 queries would take all 256 VGPRs) a 32-query half of one; a block covers
-// kDqW waves' queries, i.e. a whole dS run (kQB tiles) or half of one
+// queries per dQ wave in full grids (QW)
 template <int D> constexpr int dq_qw() { return D == 256 ? 32 : 64; }
 
 template <int D, int QW> struct DqSmem {
@@ -1201,10 +1202,11 @@ __global__ __launch_bounds__(512, D == 64 && KR == 32 ? 4 : 1) void attn_bwd_dkv
   if (n_it > 0) issue(0, qbase);
   if (prole) dma_wait();
   __syncthreads();
-  // D role: dP of the current and the next chunk. Computed ahead only where one
-  // block's two waves per SIMD run alone and the registers are there (D = 32 and
-  // 128, 32 keys per wave): with two blocks per CU (D = 64, 128 registers) the
-  // look-ahead would spill, and at 16 keys per wave it does in the
+  // D role: dP of the current and the next chunk. Computed ahead where the
+  // registers are there: 32 keys per wave at D = 128 (one block per CU) and D = 32
+  // (121-129 registers with it: two blocks per CU but for the non-causal mode
+  // with a padding mask, whose 129 leave one). In the 128 registers of D = 64
+  // the look-ahead would spill, and at 16 keys per wave it does in the
   // non-causal modes (D = 256 measured 0-3% faster causal and 8% non-causal
   // without, bit-identical); dP is then computed after the barrier, half by half
   constexpr bool kAhead = KS == 2 && D != 64;
@@ -1506,10 +1508,11 @@ template <typename T, int D, int DE, int MODE> int launch_fwd(const AttnArgs& a,
   return check_launch("kat_attn_fwd (mfma)");
 }
 
-// Small grids. A dK/dV block is one per CU and walks every query chunk of its
-// keys, a dQ block every key stage of its queries; while the grid is short of
-// the chip, the time is that of the longest block's chain, and fewer rows per
-// wave (16 keys, 32 queries) make its steps shorter and the blocks more.
+// Small grids. A dK/dV block walks every query chunk of its keys, a dQ block
+// every key stage of its queries; while the grid is short of the chip (a CU
+// holds one dK/dV block at D = 128 and two at D <= 64, one dQ block), the time is
+// that of the longest block's chain, and fewer rows per wave (16 keys, 32
+// queries) make its steps shorter and the blocks more.
 // Results are the same bits in causal mode (dK/dV rows are summed over
 // the queries in the same order, dQ rows over the keys).
 // dK/dV with 16 keys per wave pair instead of 32, nb: blocks of 128 keys. It reads

@@ -313,10 +313,11 @@ def test_mfma_backward_key_groups_of_different_magnitude(gpu, D, dtype, width, m
     # cycles 2^s, 1, 2^-s from one group of `width` keys to the next give every
     # 32-key group a different exponent (also inside each 64-key tile): a wrong
     # exponent for any group would move that group's share of dq or dk by 2^s.
-    # width 16: the two 16-key halves of a 32-key group differ (at D = 256 two
-    # wave pairs own them and must agree on the group's exponent: one from
-    # the smaller half would overflow the larger half's fp16 copy). At D = 64
-    # one wave pair owns 64 keys, two groups with an exponent each.
+    # width 16: the two 16-key halves of a 32-key group differ. In a grid of this
+    # size (and at D = 256 in any) a wave pair owns 16 keys: two pairs must agree
+    # on their group's exponent, or one from the smaller half would overflow the
+    # larger half's fp16 copy. Full grids, where a pair owns the group, are in
+    # test_gpu_attention_full_grids.py.
     _pin_mfma(monkeypatch, D)
     B, H, T = 1, 2, 300
     q, k, v, do = (t.float() for t in _inputs(47 + D, B, H, T, D, torch.float32))
